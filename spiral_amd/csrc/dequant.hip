@@ -28,16 +28,17 @@ namespace {
 constexpr int kDequantGroups = 512;
 template <int TYPE>
 __global__ void __launch_bounds__(256) dequant_kernel(const uint8_t* __restrict__ w, int64_t n_rows,
-                                                      int64_t nb, uint32_t groups_per_row, uint32_t wg_per_row,
-                                                      uint16_t* __restrict__ out, int64_t ld_out) {
+                                                      int64_t nb, int64_t row0, uint32_t groups_per_row,
+                                                      uint32_t wg_per_row, uint16_t* __restrict__ out,
+                                                      int64_t ld_out) {
   const uint32_t row = blockIdx.x / wg_per_row;
   const uint32_t g0 = (blockIdx.x - row * wg_per_row) * kDequantGroups + threadIdx.x;
   if (g0 >= groups_per_row) return;
   const uint32_t g1 = g0 + 256;
   const bool second = g1 < groups_per_row;
   float v[2][8];
-  dequant8<TYPE>(w, n_rows, nb, row, g0, v[0]);
-  dequant8<TYPE>(w, n_rows, nb, row, second ? g1 : g0, v[1]);
+  dequant8<TYPE>(w, n_rows, nb, row0 + row, g0, v[0]);
+  dequant8<TYPE>(w, n_rows, nb, row0 + row, second ? g1 : g0, v[1]);
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
     if (h == 1 && !second) break;
@@ -82,6 +83,31 @@ __global__ void __launch_bounds__(256) get_rows_kernel(const uint8_t* __restrict
 }
 
 }  // namespace
+
+// Rows row0 .. row0 + rows - 1 of an n_rows x k matrix -> bf16 rows of out;
+// arguments validated by the caller.
+int dequant_rows(int type, const void* w, int64_t n_rows, int64_t k, int64_t row0, int64_t rows, uint16_t* out,
+                 int64_t ld_out, hipStream_t s) {
+  const int64_t nb = k / block_elems(type), gpr = k / 8, wpr = ceil_div(gpr, kDequantGroups);
+  if (gpr + 256 > UINT32_MAX || rows > UINT32_MAX || rows * wpr > UINT32_MAX) return SPIRAL_ERR_SHAPE;
+  const dim3 grid(static_cast<unsigned>(rows * wpr));
+  const uint32_t g32 = static_cast<uint32_t>(gpr), w32 = static_cast<uint32_t>(wpr);
+  const uint8_t* W = static_cast<const uint8_t*>(w);
+#define SPIRAL_DEQUANT(T) \
+  hipLaunchKernelGGL(dequant_kernel<T>, grid, dim3(256), 0, s, W, n_rows, nb, row0, g32, w32, out, ld_out)
+  switch (type) {
+    case SPIRAL_TYPE_Q4_0: SPIRAL_DEQUANT(SPIRAL_TYPE_Q4_0); break;
+    case SPIRAL_TYPE_Q8_0: SPIRAL_DEQUANT(SPIRAL_TYPE_Q8_0); break;
+    case SPIRAL_TYPE_Q4_K: SPIRAL_DEQUANT(SPIRAL_TYPE_Q4_K); break;
+    case SPIRAL_TYPE_Q5_K: SPIRAL_DEQUANT(SPIRAL_TYPE_Q5_K); break;
+    case SPIRAL_TYPE_IQ4_NL: SPIRAL_DEQUANT(SPIRAL_TYPE_IQ4_NL); break;
+    case SPIRAL_TYPE_IQ4_XS: SPIRAL_DEQUANT(SPIRAL_TYPE_IQ4_XS); break;
+    default: SPIRAL_DEQUANT(SPIRAL_TYPE_Q6_K); break;
+  }
+#undef SPIRAL_DEQUANT
+  return launch_status();
+}
+
 }  // namespace spiral
 
 using namespace spiral;
@@ -96,25 +122,7 @@ int spiral_dequant_bf16(int type, const void* w, int64_t n_rows, int64_t k, uint
   if (!aligned16(w) || !aligned16(out) || ld_out % 8 != 0) return SPIRAL_ERR_ALIGN;
   int rc = require_device();
   if (rc != SPIRAL_OK) return rc;
-  const int64_t nb = k / block_elems(type), gpr = k / 8, wpr = ceil_div(gpr, kDequantGroups);
-  if (gpr + 256 > UINT32_MAX || n_rows > UINT32_MAX || n_rows * wpr > UINT32_MAX) return SPIRAL_ERR_SHAPE;
-  const dim3 grid(static_cast<unsigned>(n_rows * wpr));
-  const uint32_t g32 = static_cast<uint32_t>(gpr), w32 = static_cast<uint32_t>(wpr);
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  const uint8_t* W = static_cast<const uint8_t*>(w);
-#define SPIRAL_DEQUANT(T) \
-  hipLaunchKernelGGL(dequant_kernel<T>, grid, dim3(256), 0, s, W, n_rows, nb, g32, w32, out, ld_out)
-  switch (type) {
-    case SPIRAL_TYPE_Q4_0: SPIRAL_DEQUANT(SPIRAL_TYPE_Q4_0); break;
-    case SPIRAL_TYPE_Q8_0: SPIRAL_DEQUANT(SPIRAL_TYPE_Q8_0); break;
-    case SPIRAL_TYPE_Q4_K: SPIRAL_DEQUANT(SPIRAL_TYPE_Q4_K); break;
-    case SPIRAL_TYPE_Q5_K: SPIRAL_DEQUANT(SPIRAL_TYPE_Q5_K); break;
-    case SPIRAL_TYPE_IQ4_NL: SPIRAL_DEQUANT(SPIRAL_TYPE_IQ4_NL); break;
-    case SPIRAL_TYPE_IQ4_XS: SPIRAL_DEQUANT(SPIRAL_TYPE_IQ4_XS); break;
-    default: SPIRAL_DEQUANT(SPIRAL_TYPE_Q6_K); break;
-  }
-#undef SPIRAL_DEQUANT
-  return launch_status();
+  return dequant_rows(type, w, n_rows, k, 0, n_rows, out, ld_out, static_cast<hipStream_t>(stream));
 }
 
 int spiral_get_rows(int type, const void* w, int64_t n_rows, int64_t k, const int32_t* ids,

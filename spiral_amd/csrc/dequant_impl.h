@@ -200,6 +200,12 @@ __device__ __forceinline__ uint32_t bload1(__amdgpu_buffer_rsrc_t r, uint32_t vo
   return __builtin_amdgcn_raw_buffer_load_b8(r, voff, soff, 0);
 }
 
+// 16 bytes a lane straight into LDS: the wave's 1 KiB lands at `lds` (wave-
+// uniform) in lane order, wherever the lanes' offsets point.
+__device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t r, void* lds, uint32_t voff, uint32_t soff) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 16, voff, soff, 0, 0);
+}
+
 // Q4_0: piece 2b + h of a row is nibble h of block b's 16 qs bytes.
 template <>
 struct Piece<SPIRAL_TYPE_Q4_0> {

@@ -1,0 +1,81 @@
+"""GPU parity of the many-row products that dequantize the weights once into
+the workspace (spiral_amd/csrc/gemm_dense.hip): every tile the dispatch
+chooses, ragged rows of x and of W, one to eighteen k steps of 64 (the LDS
+stages' prologue and the F32 accumulator flush), strided and misaligned
+outputs, the fused fallback, and a matrix taken in two chunks. Held to the
+product bars of tests/test_gpu_parity.py against the float64 oracle.
+"""
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import oracle as O
+from spiral_amd import lib, ops, synth
+from test_gpu_parity import REL_TOL, REL_TOL_EXACT_W, _mul_mat_case, dev_bf16, dev_u8, rel_err
+
+pytestmark = pytest.mark.gpu
+
+# One row or more past whole tiles in both directions; the tile widths follow
+# from the sizes (128 x 128, 256 x 128, .. 256 x 256).
+SHAPES = [
+    (O.Q4_0, 257, 7001, 64),
+    (O.Q4_0, 1300, 1501, 96 * 12),
+    (O.Q8_0, 769, 5003, 128),
+    (O.Q5_K, 1025, 7001, 256),
+    (O.IQ4_NL, 1300, 7001, 192),
+    (O.IQ4_XS, 1537, 7001, 256),
+    (O.Q6_K, 2049, 7001, 256),
+    (O.Q4_K, 513, 7001, 1024),
+]
+
+
+def takes_dense(qtype, m, n, k):
+    return lib().spiral_mul_mat_workspace_bytes(qtype, n, k, m) == n * k * 2
+
+
+@pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("qtype,m,n,k", SHAPES)
+def test_dense_tiles(cuda, qtype, m, n, k, out_dtype):
+    assert takes_dense(qtype, m, n, k)
+    y, ref = _mul_mat_case(cuda, qtype, n, k, m, 200, out_dtype)
+    assert rel_err(y, ref) <= (REL_TOL if out_dtype == torch.bfloat16 else REL_TOL_EXACT_W)
+
+
+@pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32])
+def test_dense_strides_and_fallback(cuda, out_dtype):
+    """x and y wider than k and n, y rows off 16-byte alignment; a workspace
+    of the packed x alone still runs (the fused GEMM), and agrees."""
+    qtype, m, n, k = O.Q8_0, 513, 5003, 128
+    assert takes_dense(qtype, m, n, k)
+    raw = synth.make_weights(qtype, n, k, 210)
+    x = synth.make_x(m, k, 211)
+    w = ops.to_planar(qtype, dev_u8(raw, cuda), n, k)
+    xw = torch.full((m, k + 40), float("nan"), dtype=torch.bfloat16, device=cuda)
+    xw[:, :k] = dev_bf16(x, cuda)
+    ref = O.matmul_f64(O.dequant(qtype, raw, n, k), x)
+    tol = REL_TOL if out_dtype == torch.bfloat16 else REL_TOL_EXACT_W
+    off = 2  # elements: 4 or 8 bytes
+    for ws in (None, torch.empty(-(-m // 16) * 16 * k * 2, dtype=torch.uint8, device=cuda)):
+        flat = torch.full((m * (n + 13) + off,), 7.0, dtype=out_dtype, device=cuda)
+        yw = flat[off:].view(m, n + 13)
+        ops.mul_mat(qtype, w, n, k, xw[:, :k], out=yw[:, :n], workspace=ws)
+        torch.cuda.synchronize()
+        got = yw.float().cpu().numpy()
+        assert rel_err(got[:, :n], ref) <= tol
+        assert (got[:, n:] == 7.0).all() and (flat[:off] == 7.0).all()  # nothing written outside
+
+
+def test_dense_chunks(cuda):
+    """A matrix above the workspace's 256 MiB of bf16: rows on both sides of
+    the chunk boundary (4352) and the last ones."""
+    qtype, m, n, k = O.Q4_K, 1500, 8500, 16384
+    assert lib().spiral_mul_mat_workspace_bytes(qtype, n, k, m) == 4352 * k * 2
+    raw = synth.make_weights(qtype, n, k, 220)
+    x = synth.make_x(m, k, 221)
+    w = ops.to_planar(qtype, dev_u8(raw, cuda), n, k)
+    y = ops.mul_mat(qtype, w, n, k, dev_bf16(x, cuda), out_dtype=torch.float32).cpu().numpy()
+    rows = np.r_[0:4, 4348:4356, 8496:8500]
+    sub = np.ascontiguousarray(raw.reshape(n, -1)[rows]).reshape(-1)
+    ref = O.matmul_f64(O.dequant(qtype, sub, len(rows), k), x)
+    assert rel_err(y[:, rows], ref) <= REL_TOL_EXACT_W
