@@ -191,8 +191,10 @@ int spiral_get_rows(int type, const void* w, int64_t n_rows, int64_t k,
  * spiral_mul_mat_workspace_bytes() bytes, which is 0 for m <= 16, in which
  * case workspace may be NULL); from a few hundred rows, where that is
  * faster, it dequantizes the matrix into `workspace` once instead (up to
- * 256 MiB at a time). A workspace of only the rewritten x (m rounded up to
- * 16, times k, 2 bytes each) is accepted too and runs the former. A workspace must not be shared by calls in
+ * 256 MiB at a time), and long rows that leave CUs idle are multiplied in
+ * ranges of k whose F32 sums go through `workspace`. A workspace of only the
+ * rewritten x (m rounded up to 16, times k, 2 bytes each) is accepted too
+ * and runs without either. A workspace must not be shared by calls in
  * flight at the same time. The small-batch form needs y within 2 GiB
  * ((m - 1) * ldy + n_rows elements), else SPIRAL_ERR_SHAPE. */
 int64_t spiral_mul_mat_workspace_bytes(int type, int64_t n_rows, int64_t k,

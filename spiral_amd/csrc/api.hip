@@ -7,10 +7,11 @@ namespace spiral {
 int64_t gemv_max_k(int type, bool exact);
 int gemv(int type, const void* w, int64_t n_rows, int64_t k, const uint16_t* x, void* y, int y_type, bool exact,
          hipStream_t s);
-int64_t gemm_workspace_bytes(int64_t m, int64_t k);
+int64_t gemm_min_workspace_bytes(int64_t m, int64_t k);
+int64_t gemm_workspace_bytes(int64_t m, int64_t n_rows, int64_t k);
 int64_t gemm_max_k();
 int gemm(int type, const void* w, int64_t n_rows, int64_t k, const uint16_t* x, int64_t ldx, int64_t m,
-         void* y, int y_type, int64_t ldy, void* workspace, hipStream_t s);
+         void* y, int y_type, int64_t ldy, void* workspace, int64_t workspace_bytes, hipStream_t s);
 bool dense_fits(int type, int64_t n_rows, int64_t k, int64_t m, int64_t ldx, bool f32);
 int64_t dense_workspace_bytes(int64_t n_rows, int64_t k);
 int gemm_dense(int type, const void* w, int64_t n_rows, int64_t k, const uint16_t* x, int64_t ldx, int64_t m, void* y,
@@ -66,7 +67,7 @@ int64_t spiral_mul_mat_workspace_bytes(int type, int64_t n_rows, int64_t k, int6
   if (!is_quant_type(type) || n_rows <= 0 || m <= 0 || k <= 0 || k % block_elems(type) != 0) return 0;
   if (m == 1 && k <= gemv_max_k(type, true)) return 0;
   if (skinny_fits(type, n_rows, k, m)) return 0;
-  const int64_t need = gemm_workspace_bytes(m, k);  // 0 past the GEMM's longest row: spiral_mul_mat refuses that shape
+  const int64_t need = gemm_workspace_bytes(m, n_rows, k);  // 0 past the GEMM's longest row: spiral_mul_mat refuses that shape
   const bool dense = need > 0 && (dense_fits(type, n_rows, k, m, k, false) || dense_fits(type, n_rows, k, m, k, true));
   return dense ? std::max(need, dense_workspace_bytes(n_rows, k)) : need;
 }
@@ -85,7 +86,7 @@ int spiral_mul_mat(int type, const void* w, int64_t n_rows, int64_t k, const uin
   if (!direct && k > gemm_max_k()) return SPIRAL_ERR_SHAPE;
   // The least workspace a call takes is the fused GEMM's; the forms that want
   // more run when the caller's workspace holds it.
-  const int64_t need = direct ? 0 : gemm_workspace_bytes(m, k);
+  const int64_t need = direct ? 0 : gemm_min_workspace_bytes(m, k);
   if (need > 0) {
     if (workspace == nullptr) return SPIRAL_ERR_NULL;
     if (workspace_bytes < need) return SPIRAL_ERR_CAPACITY;
@@ -101,7 +102,7 @@ int spiral_mul_mat(int type, const void* w, int64_t n_rows, int64_t k, const uin
   if (dense_fits(type, n_rows, k, m, ldx, y_type == SPIRAL_TYPE_F32) &&
       workspace_bytes >= dense_workspace_bytes(n_rows, k))
     return gemm_dense(type, w, n_rows, k, x, ldx, m, y, y_type, ldy, workspace, s);
-  return gemm(type, w, n_rows, k, x, ldx, m, y, y_type, ldy, workspace, s);
+  return gemm(type, w, n_rows, k, x, ldx, m, y, y_type, ldy, workspace, workspace_bytes, s);
 }
 
 int64_t spiral_gemv_relaxed_max_k(int type) { return is_quant_type(type) ? gemv_max_k(type, false) : 0; }

@@ -128,7 +128,8 @@ __device__ __forceinline__ void dequant8(const uint8_t* __restrict__ w, int64_t 
 // Pieces are read with buffer loads: Piece::Addr fixes, per thread, the row
 // and the piece's place inside a 128-element k step (pl = 0..7), and a step
 // adds only scalar offsets. Offsets are 32-bit, so every plane of the
-// weight tensor must stay below 4 GiB (checked by the launcher).
+// weight tensor must stay below 4 GiB (checked by the launcher). Piece::skip
+// moves an Addr on by an even number of 128-element steps.
 //
 // The values equal dequant8's. The one difference is the sign of a zero
 // weight (code 8 of Q4_0, 0 of Q8_0, 32 of Q6_K) under a negative scale: +0
@@ -220,6 +221,7 @@ struct Piece<SPIRAL_TYPE_Q4_0> {
     const uint32_t b = static_cast<uint32_t>(n * nb) + (pl >> 1);
     return Addr{b * 16u, b * 2u, pl & 1};
   }
+  static __device__ __forceinline__ void skip(Addr& a, uint32_t steps) { a.qs += steps * 64u, a.d += steps * 8u; }
   // Step starting at element k0 (a multiple of 128).
   __device__ __forceinline__ void load(const Planes& P, const Addr& A, int64_t k0) {
     const uint32_t kb = static_cast<uint32_t>(k0 >> 5);
@@ -262,6 +264,7 @@ struct Piece<SPIRAL_TYPE_Q8_0> {
     const uint32_t b = static_cast<uint32_t>(n * nb) + (pl >> 1);
     return Addr{b * 32u + 16u * (pl & 1), b * 2u};
   }
+  static __device__ __forceinline__ void skip(Addr& a, uint32_t steps) { a.qs += steps * 128u, a.d += steps * 8u; }
   __device__ __forceinline__ void load(const Planes& P, const Addr& A, int64_t k0) {
     const uint32_t kb = static_cast<uint32_t>(k0 >> 5);
     q = bload16(P.a, A.qs, kb * 32u);
@@ -301,6 +304,9 @@ struct Piece<SPIRAL_TYPE_Q6_K> {
     const int j = pl >> 1, l0 = 16 * (pl & 1);
     return Addr{blk * 128u + 32u * (j & 1) + l0, blk * 64u + l0, blk * 16u + (pl & 1) + 2 * j, blk * 2u,
                 (j >> 1) * 4, 2 * j};
+  }
+  static __device__ __forceinline__ void skip(Addr& a, uint32_t steps) {
+    a.ql += steps * 64u, a.qh += steps * 32u, a.sc += steps * 8u, a.d += steps;
   }
   __device__ __forceinline__ void load(const Planes& P, const Addr& A, int64_t k0) {
     const uint32_t sb = static_cast<uint32_t>(k0 >> 8), h = static_cast<uint32_t>((k0 >> 7) & 1);
@@ -347,6 +353,9 @@ struct PieceKQ {
     const uint32_t blk = static_cast<uint32_t>(n * nb);
     return Addr{blk * 128u + 32u * (pl >> 2) + 16u * (pl & 1), blk * 32u + 16u * (pl & 1), blk * 16u, pl >> 1,
                 (pl >> 1) & 1};
+  }
+  static __device__ __forceinline__ void skip(Addr& a, uint32_t steps) {
+    a.qs += steps * 64u, a.qh += steps * 16u, a.meta += steps * 8u;
   }
   __device__ __forceinline__ void load(const Planes& P, const Addr& A, int64_t k0) {
     const uint32_t sb = static_cast<uint32_t>(k0 >> 8), h = static_cast<uint32_t>((k0 >> 7) & 1);
@@ -408,6 +417,7 @@ struct Piece<SPIRAL_TYPE_IQ4_NL> {
   static __device__ __forceinline__ Addr addr(int64_t n, int64_t nb, int pl) {
     return Piece<SPIRAL_TYPE_Q4_0>::addr(n, nb, pl);
   }
+  static __device__ __forceinline__ void skip(Addr& a, uint32_t steps) { Piece<SPIRAL_TYPE_Q4_0>::skip(a, steps); }
   __device__ __forceinline__ void load(const Planes& P, const Addr& A, int64_t k0) {
     const uint32_t kb = static_cast<uint32_t>(k0 >> 5);
     q = bload16(P.a, A.qs, kb * 16u);
@@ -434,6 +444,7 @@ struct Piece<SPIRAL_TYPE_IQ4_XS> {
     const uint32_t blk = static_cast<uint32_t>(n * nb);
     return Addr{blk * 128u + 16u * (pl >> 1), blk * 8u, pl >> 1, pl & 1};
   }
+  static __device__ __forceinline__ void skip(Addr& a, uint32_t steps) { a.qs += steps * 64u, a.meta += steps * 4u; }
   __device__ __forceinline__ void load(const Planes& P, const Addr& A, int64_t k0) {
     const uint32_t sb = static_cast<uint32_t>(k0 >> 8), h = static_cast<uint32_t>((k0 >> 7) & 1);
     q = bload16(P.a, A.qs, sb * 128u + 64u * h);

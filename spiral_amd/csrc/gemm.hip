@@ -44,6 +44,7 @@
 
 namespace spiral {
 int64_t gemm_max_k();
+int64_t gemm_workspace_bytes(int64_t m, int64_t n_rows, int64_t k);
 
 namespace {
 
@@ -170,7 +171,8 @@ __device__ __forceinline__ void gemm_step(f32x4_t (&acc)[4][4], Pipe<TYPE>& pp, 
 template <int TYPE, bool F32_OUT>
 __global__ void __launch_bounds__(kThreads) gemm_kernel(const uint8_t* __restrict__ w, int64_t n_rows, int64_t k,
                                                         const uint16_t* __restrict__ xp, int64_t m,
-                                                        void* __restrict__ y, int64_t ldy, int64_t n_tiles_n) {
+                                                        void* __restrict__ y, int64_t ldy, int64_t n_tiles_n,
+                                                        int64_t y_split) {
   // Four weight tiles during the loop; the k-quarter partial sums after it.
   __shared__ __align__(16) float smem[kRedFloats];
   uint16_t* Bs = reinterpret_cast<uint16_t*>(smem);
@@ -183,17 +185,24 @@ __global__ void __launch_bounds__(kThreads) gemm_kernel(const uint8_t* __restric
   const int64_t nb = k / block_elems(TYPE);
   // 32-bit step counters keep the ring's clamps scalar (k is at most
   // gemm_max_k(), so k / 128 fits)
-  const int full = static_cast<int>(k / kBK);
-  const int tail = static_cast<int>(k - full * kBK);  // 0, 32, 64 or 96
-
+  // Workgroup (b, z) of Z = gridDim.y takes the z-th of Z ranges of k steps
+  // (whole pairs of steps: super-blocks), `full` steps from step kb, and writes
+  // to y + z * y_split; the last range has the k tail. The range's start goes
+  // into the lanes' offsets, so the loop counts from 0.
+  const int all = static_cast<int>(k / kBK), z = blockIdx.y, nz = gridDim.y;
+  const int kb = static_cast<int>(static_cast<int64_t>(all / 2) * z / nz) * 2;
+  const bool last = z + 1 == nz;
+  const int full = (last ? all : static_cast<int>(static_cast<int64_t>(all / 2) * (z + 1) / nz) * 2) - kb;
+  const int tail = last ? static_cast<int>(k - static_cast<int64_t>(all) * kBK) : 0;  // 0, 32, 64 or 96
   const int64_t kk_n = k >> 5, mb_n = (m + 15) >> 4;
   const __amdgpu_buffer_rsrc_t X = buffer_rsrc(xp, static_cast<uint32_t>(mb_n * kk_n * 1024));
   uint32_t voff[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i)
-    voff[i] = static_cast<uint32_t>(min((row0 >> 4) + i, mb_n - 1) * kk_n * 1024 + lane * 16);
+    voff[i] = static_cast<uint32_t>((min((row0 >> 4) + i, mb_n - 1) * kk_n + 4 * kb) * 1024 + lane * 16);
   const Planes P = make_planes<TYPE>(w, n_rows, nb);
-  const typename Piece<TYPE>::Addr pa = Piece<TYPE>::addr(min(n0 + (tid >> 3), n_rows - 1), nb, tid & 7);
+  typename Piece<TYPE>::Addr pa = Piece<TYPE>::addr(min(n0 + (tid >> 3), n_rows - 1), nb, tid & 7);
+  Piece<TYPE>::skip(pa, static_cast<uint32_t>(kb));
 
   f32x4_t acc[4][4];
 #pragma unroll
@@ -294,7 +303,7 @@ __global__ void __launch_bounds__(kThreads) gemm_kernel(const uint8_t* __restric
     const int64_t gm = row0 + 16 * q + r, gn = n0 + col;
     if (gm >= m) continue;
     const uint4 v = *reinterpret_cast<const uint4*>(T + r * kTPitch + col);
-    OutT* dst = static_cast<OutT*>(y) + gm * ldy + gn;
+    OutT* dst = static_cast<OutT*>(y) + z * y_split + gm * ldy + gn;
     if (gn + kPer <= n_rows && (reinterpret_cast<uintptr_t>(dst) & 15u) == 0) {
       *reinterpret_cast<uint4*>(dst) = v;
     } else {
@@ -304,14 +313,61 @@ __global__ void __launch_bounds__(kThreads) gemm_kernel(const uint8_t* __restric
   }
 }
 
+// y[r][c] = sum over z of part[z][r][c] (r < m, c < n, z < nz, n a multiple of
+// 4), in z order: a thread takes four columns.
+template <bool F32_OUT>
+__global__ void __launch_bounds__(256) sum_splits_kernel(const float* __restrict__ part, int nz, int64_t m, int64_t n,
+                                                         void* __restrict__ y, int64_t ldy) {
+  const int64_t i = 4 * (static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x);
+  if (i >= m * n) return;
+  f32x4_t v = *reinterpret_cast<const f32x4_t*>(part + i);
+  for (int z = 1; z < nz; ++z) v += *reinterpret_cast<const f32x4_t*>(part + z * m * n + i);
+  const int64_t r = i / n, c = i - r * n;
+  if constexpr (F32_OUT) {
+    float* dst = static_cast<float*>(y) + r * ldy + c;
+    if ((reinterpret_cast<uintptr_t>(dst) & 15u) == 0) {
+      *reinterpret_cast<f32x4_t*>(dst) = v;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) dst[e] = v[e];
+    }
+  } else {
+    uint16_t* dst = static_cast<uint16_t*>(y) + r * ldy + c;
+    const uint32_t lo = pack_bf16x2(v[0], v[1]), hi = pack_bf16x2(v[2], v[3]);
+    if ((reinterpret_cast<uintptr_t>(dst) & 7u) == 0) {
+      *reinterpret_cast<uint2*>(dst) = make_uint2(lo, hi);
+    } else {
+      const uint32_t w[2] = {lo, hi};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) dst[e] = static_cast<uint16_t>(w[e / 2] >> (16 * (e & 1)));
+    }
+  }
+}
+
 // Rows of X per launch: the packed chunk (rows rounded up to 16, times k
 // bf16) stays below 2 GiB so buffer offsets fit in 32 bits.
 // k is at most gemm_max_k(), so one M tile of packed X fits.
 int64_t chunk_rows(int64_t k) { return std::max<int64_t>(kBM, (kMaxBufferBytes / (k * 2)) / kBM * kBM); }
 
+int64_t packed_bytes(int64_t m, int64_t k) { return ceil_div(std::min(m, chunk_rows(k)), 16) * 16 * k * 2; }
+
+// Ranges of k that share the tiles' work when the tiles leave CUs idle. The
+// ranges' F32 sums go through the workspace and are added by a second launch
+// (about 4 us), so a range keeps at least 2048 of k, and the sums at most 2.5
+// times the bytes of the packed x: long rows (a down projection) split, square
+// projections do not. Q5_K, us, one range against the split: 4096 x 14336, 77 rows
+// (64 tiles, four ranges) 73 and 31, 250 rows (two) 79 and 52; 2048 x 8192, 77
+// rows 45 and 21; 1024 x 4096, 250 rows 28 and 21.
+int64_t k_splits(int64_t m, int64_t n_rows, int64_t k) {
+  if (m > chunk_rows(k) || n_rows % 4 != 0) return 1;
+  const int64_t tiles = ceil_div(m, kBM) * ceil_div(n_rows, kBN);
+  const int64_t nz = std::min(std::min<int64_t>(device_cu_count() / tiles, k / 2048), 5 * k / (4 * n_rows));
+  return std::max<int64_t>(1, std::min<int64_t>(nz, 8));
+}
+
 template <int TYPE>
 int launch_gemm(const void* w, int64_t n_rows, int64_t k, const uint16_t* x, int64_t ldx, int64_t m, void* y,
-                int y_type, int64_t ldy, uint16_t* xp, hipStream_t s) {
+                int y_type, int64_t ldy, uint16_t* xp, int64_t workspace_bytes, hipStream_t s) {
   // Weight planes are addressed with 32-bit offsets (the largest plane is at
   // most 16/18 of the tensor).
   const int64_t wbytes = spiral_tensor_bytes(TYPE, n_rows, k);
@@ -331,10 +387,23 @@ int launch_gemm(const void* w, int64_t n_rows, int64_t k, const uint16_t* x, int
     if (rc != SPIRAL_OK) return rc;
     const dim3 grid(static_cast<unsigned>(tn * tm));
     void* yc = static_cast<uint8_t*>(y) + mo * ldy * ysz;
-    if (y_type == SPIRAL_TYPE_F32)
-      hipLaunchKernelGGL((gemm_kernel<TYPE, true>), grid, dim3(kThreads), 0, s, W, n_rows, k, xp, mc, yc, ldy, tn);
-    else
-      hipLaunchKernelGGL((gemm_kernel<TYPE, false>), grid, dim3(kThreads), 0, s, W, n_rows, k, xp, mc, yc, ldy, tn);
+    const int64_t nz = k_splits(m, n_rows, k);
+    if (nz > 1 && workspace_bytes >= gemm_workspace_bytes(m, n_rows, k)) {  // one chunk
+      float* part = reinterpret_cast<float*>(reinterpret_cast<uint8_t*>(xp) + packed_bytes(m, k));
+      hipLaunchKernelGGL((gemm_kernel<TYPE, true>), dim3(grid.x, static_cast<unsigned>(nz)), dim3(kThreads), 0, s, W,
+                         n_rows, k, xp, m, part, n_rows, tn, m * n_rows);
+      rc = launch_status();
+      if (rc != SPIRAL_OK) return rc;
+      const dim3 sums(static_cast<unsigned>(ceil_div(m * n_rows, 1024)));
+      if (y_type == SPIRAL_TYPE_F32)
+        hipLaunchKernelGGL(sum_splits_kernel<true>, sums, dim3(256), 0, s, part, static_cast<int>(nz), m, n_rows, y, ldy);
+      else
+        hipLaunchKernelGGL(sum_splits_kernel<false>, sums, dim3(256), 0, s, part, static_cast<int>(nz), m, n_rows, y, ldy);
+    } else if (y_type == SPIRAL_TYPE_F32) {
+      hipLaunchKernelGGL((gemm_kernel<TYPE, true>), grid, dim3(kThreads), 0, s, W, n_rows, k, xp, mc, yc, ldy, tn, 0);
+    } else {
+      hipLaunchKernelGGL((gemm_kernel<TYPE, false>), grid, dim3(kThreads), 0, s, W, n_rows, k, xp, mc, yc, ldy, tn, 0);
+    }
     rc = launch_status();
     if (rc != SPIRAL_OK) return rc;
   }
@@ -347,27 +416,30 @@ int launch_gemm(const void* w, int64_t n_rows, int64_t k, const uint16_t* x, int
 // 32-bit buffer offset.
 int64_t gemm_max_k() { return kMaxBufferBytes / (2 * kBM); }
 
-// Workspace for the packed X of one launch chunk (0 when k > gemm_max_k()).
-int64_t gemm_workspace_bytes(int64_t m, int64_t k) {
+// Least workspace: the packed X of one launch chunk (0 when k > gemm_max_k()).
+int64_t gemm_min_workspace_bytes(int64_t m, int64_t k) { return k <= 0 || k > gemm_max_k() ? 0 : packed_bytes(m, k); }
+
+// With room for the sums of k ranges where the product splits.
+int64_t gemm_workspace_bytes(int64_t m, int64_t n_rows, int64_t k) {
   if (k <= 0 || k > gemm_max_k()) return 0;
-  const int64_t rows = std::min(m, chunk_rows(k));
-  return ceil_div(rows, 16) * 16 * k * 2;
+  const int64_t nz = k_splits(m, n_rows, k);
+  return packed_bytes(m, k) + (nz > 1 ? nz * m * n_rows * 4 : 0);
 }
 
 // Y = X W^T; arguments validated by the caller (k a multiple of the block, x
 // rows 16-byte aligned with ldx a multiple of 8, workspace of at least
-// gemm_workspace_bytes(m, k) bytes, 16-byte aligned).
+// gemm_min_workspace_bytes(m, k) bytes, 16-byte aligned).
 int gemm(int type, const void* w, int64_t n_rows, int64_t k, const uint16_t* x, int64_t ldx, int64_t m, void* y,
-         int y_type, int64_t ldy, void* workspace, hipStream_t s) {
+         int y_type, int64_t ldy, void* workspace, int64_t workspace_bytes, hipStream_t s) {
   uint16_t* xp = static_cast<uint16_t*>(workspace);
   switch (type) {
-    case SPIRAL_TYPE_Q4_0: return launch_gemm<SPIRAL_TYPE_Q4_0>(w, n_rows, k, x, ldx, m, y, y_type, ldy, xp, s);
-    case SPIRAL_TYPE_Q8_0: return launch_gemm<SPIRAL_TYPE_Q8_0>(w, n_rows, k, x, ldx, m, y, y_type, ldy, xp, s);
-    case SPIRAL_TYPE_Q6_K: return launch_gemm<SPIRAL_TYPE_Q6_K>(w, n_rows, k, x, ldx, m, y, y_type, ldy, xp, s);
-    case SPIRAL_TYPE_Q4_K: return launch_gemm<SPIRAL_TYPE_Q4_K>(w, n_rows, k, x, ldx, m, y, y_type, ldy, xp, s);
-    case SPIRAL_TYPE_Q5_K: return launch_gemm<SPIRAL_TYPE_Q5_K>(w, n_rows, k, x, ldx, m, y, y_type, ldy, xp, s);
-    case SPIRAL_TYPE_IQ4_NL: return launch_gemm<SPIRAL_TYPE_IQ4_NL>(w, n_rows, k, x, ldx, m, y, y_type, ldy, xp, s);
-    case SPIRAL_TYPE_IQ4_XS: return launch_gemm<SPIRAL_TYPE_IQ4_XS>(w, n_rows, k, x, ldx, m, y, y_type, ldy, xp, s);
+    case SPIRAL_TYPE_Q4_0: return launch_gemm<SPIRAL_TYPE_Q4_0>(w, n_rows, k, x, ldx, m, y, y_type, ldy, xp, workspace_bytes, s);
+    case SPIRAL_TYPE_Q8_0: return launch_gemm<SPIRAL_TYPE_Q8_0>(w, n_rows, k, x, ldx, m, y, y_type, ldy, xp, workspace_bytes, s);
+    case SPIRAL_TYPE_Q6_K: return launch_gemm<SPIRAL_TYPE_Q6_K>(w, n_rows, k, x, ldx, m, y, y_type, ldy, xp, workspace_bytes, s);
+    case SPIRAL_TYPE_Q4_K: return launch_gemm<SPIRAL_TYPE_Q4_K>(w, n_rows, k, x, ldx, m, y, y_type, ldy, xp, workspace_bytes, s);
+    case SPIRAL_TYPE_Q5_K: return launch_gemm<SPIRAL_TYPE_Q5_K>(w, n_rows, k, x, ldx, m, y, y_type, ldy, xp, workspace_bytes, s);
+    case SPIRAL_TYPE_IQ4_NL: return launch_gemm<SPIRAL_TYPE_IQ4_NL>(w, n_rows, k, x, ldx, m, y, y_type, ldy, xp, workspace_bytes, s);
+    case SPIRAL_TYPE_IQ4_XS: return launch_gemm<SPIRAL_TYPE_IQ4_XS>(w, n_rows, k, x, ldx, m, y, y_type, ldy, xp, workspace_bytes, s);
     default: return SPIRAL_ERR_TYPE;
   }
 }
