@@ -261,13 +261,20 @@ const uint16_t* act_bf16(const spiral_tensor* b, uint8_t* scratch, bool force_co
   return dst;
 }
 
-int compute_mul_mat(spiral_backend* be, const spiral_tensor* t) {
+// held: the tensor whose bf16 copy the start of the scratch holds (null: none),
+// so that the products over one activation convert it once, or not at all when
+// the node that produced it left the copy.
+int compute_mul_mat(spiral_backend* be, const spiral_tensor* t, const spiral_tensor*& held) {
   const spiral_tensor* a = t->src[0];
   const spiral_tensor* b = t->src[1];
-  int rc;
-  int64_t ld1, ld2, ld3;
-  const uint16_t* xb = act_bf16(b, be->scratch, false, be->stream, ld1, ld2, ld3, rc);
-  if (rc != SPIRAL_OK) return rc;
+  int rc = SPIRAL_OK;
+  int64_t ld1 = b->ne[0], ld2 = ld1 * b->ne[1], ld3 = ld2 * b->ne[2];
+  const uint16_t* xb = reinterpret_cast<const uint16_t*>(be->scratch);
+  if (held != b) {
+    xb = act_bf16(b, be->scratch, false, be->stream, ld1, ld2, ld3, rc);
+    if (rc != SPIRAL_OK) return rc;
+    if (act_scratch(b) != 0) held = b;
+  }
   const int64_t r2 = b->ne[2] / a->ne[2], r3 = b->ne[3] / a->ne[3];
   uint8_t* ws = be->scratch + act_scratch(b);
   const int64_t wsb = static_cast<int64_t>(mul_mat_workspace(t));
@@ -284,7 +291,8 @@ int compute_mul_mat(spiral_backend* be, const spiral_tensor* t) {
   return SPIRAL_OK;
 }
 
-int compute_get_rows(spiral_backend* be, const spiral_tensor* t) {
+// copy (get_rows and GLU; may be null): the output as contiguous bf16 too.
+int compute_get_rows(spiral_backend* be, const spiral_tensor* t, uint16_t* copy) {
   const spiral_tensor* a = t->src[0];
   const spiral_tensor* ids = t->src[1];
   const size_t es = elem_size(t->type);
@@ -294,8 +302,9 @@ int compute_get_rows(spiral_backend* be, const spiral_tensor* t) {
       const int32_t* id = reinterpret_cast<const int32_t*>(static_cast<const uint8_t*>(ids->data) + i1 * ids->nb[1] +
                                                            i2 * ids->nb[2]);
       uint8_t* out = static_cast<uint8_t*>(t->data) + i1 * t->nb[2] + i2 * t->nb[3];
-      const int rc = spiral_get_rows(a->type, w, a->ne[1], a->ne[0], id, ids->ne[0], out, t->type,
-                                     static_cast<int64_t>(t->nb[1] / es), be->stream);
+      uint16_t* cp = copy == nullptr ? nullptr : copy + (i2 * ids->ne[1] + i1) * ids->ne[0] * t->ne[0];
+      const int rc = get_rows_copy(a->type, w, a->ne[1], a->ne[0], id, ids->ne[0], out, t->type,
+                                   static_cast<int64_t>(t->nb[1] / es), cp, be->stream);
       if (rc != SPIRAL_OK) return rc;
     }
   }
@@ -339,32 +348,25 @@ int compute_mul_mat_id_glu(spiral_backend* be, const spiral_tensor* t, const spi
 // dimensions, checked by supports_op. As in ggml, op_params[1] (swapped)
 // applies to the single-tensor form only: the split form always activates
 // src0 (ggml_glu_split sets it to 0, and ggml's kernels ignore it there).
-int compute_glu(spiral_backend* be, const spiral_tensor* t) {
+int compute_glu(spiral_backend* be, const spiral_tensor* t, uint16_t* copy) {
   const spiral_tensor* a = t->src[0];
   const spiral_tensor* b2 = t->src[1];
   const int64_t rows = t->ne[1] * t->ne[2] * t->ne[3];
-  if (t->op_params[0] == SPIRAL_GLU_SWIGLU_OAI) {
+  const int op = t->op_params[0];
+  float alpha = 0.0f, limit = 0.0f;
+  if (op == SPIRAL_GLU_SWIGLU_OAI) {
     // ggml keeps alpha and limit as floats in op_params[2] and [3].
-    float alpha, limit;
     std::memcpy(&alpha, &t->op_params[2], sizeof alpha);
     std::memcpy(&limit, &t->op_params[3], sizeof limit);
-    if (b2 != nullptr)
-      return spiral_glu_split_swiglu_oai(0, alpha, limit, static_cast<const float*>(a->data),
-                                         static_cast<int64_t>(a->nb[1] / 4), static_cast<const float*>(b2->data),
-                                         static_cast<int64_t>(b2->nb[1] / 4), t->ne[0], rows,
-                                         static_cast<float*>(t->data), static_cast<int64_t>(t->nb[1] / 4), be->stream);
-    return spiral_glu_swiglu_oai(t->op_params[1], alpha, limit, static_cast<const float*>(a->data),
-                                 static_cast<int64_t>(a->nb[1] / 4), t->ne[0], rows, static_cast<float*>(t->data),
-                                 static_cast<int64_t>(t->nb[1] / 4), be->stream);
   }
+  float* y = static_cast<float*>(t->data);
+  const int64_t ldy = static_cast<int64_t>(t->nb[1] / 4);
   if (b2 != nullptr)
-    return spiral_glu_split(t->op_params[0], 0, static_cast<const float*>(a->data),
-                            static_cast<int64_t>(a->nb[1] / 4), static_cast<const float*>(b2->data),
-                            static_cast<int64_t>(b2->nb[1] / 4), t->ne[0], rows, static_cast<float*>(t->data),
-                            static_cast<int64_t>(t->nb[1] / 4), be->stream);
-  return spiral_glu(t->op_params[0], t->op_params[1], static_cast<const float*>(a->data),
-                    static_cast<int64_t>(a->nb[1] / 4), t->ne[0], rows, static_cast<float*>(t->data),
-                    static_cast<int64_t>(t->nb[1] / 4), be->stream);
+    return glu_split_entry(op, 0, alpha, limit, static_cast<const float*>(a->data), static_cast<int64_t>(a->nb[1] / 4),
+                           static_cast<const float*>(b2->data), static_cast<int64_t>(b2->nb[1] / 4), t->ne[0], rows, y,
+                           ldy, copy, be->stream);
+  return glu_entry(op, t->op_params[1], alpha, limit, static_cast<const float*>(a->data),
+                   static_cast<int64_t>(a->nb[1] / 4), t->ne[0], rows, y, ldy, copy, be->stream);
 }
 
 // ggml's split form fused: MUL_MAT_ID over the gate experts (g->src[0]) and
@@ -437,6 +439,29 @@ bool fusable_glu_split(const spiral_cgraph* graph, int32_t i) {
       if (graph->nodes[j]->src[s] == t0 || graph->nodes[j]->src[s] == t1) return false;
   }
   return true;
+}
+
+// Where node i, a producer of F32 rows, leaves them as bf16 too: the start of
+// the scratch, if the next node multiplies them (their conversion costs a
+// launch of its own, 2.7 us and its gap for one row). Empty tensors and others
+// that the product would read in place have none.
+uint16_t* copy_for_next(const spiral_backend* be, const spiral_cgraph* graph, int32_t i) {
+  const spiral_tensor* t = graph->nodes[i];
+  if (i + 1 >= graph->n_nodes || t->type != SPIRAL_TYPE_F32) return nullptr;
+  const spiral_tensor* next = graph->nodes[i + 1];
+  if (next->op != SPIRAL_OP_MUL_MAT || next->src[1] != t) return nullptr;
+  return reinterpret_cast<uint16_t*>(be->scratch);
+}
+
+// Whether node t's output shares memory with `b` (strided extents).
+bool overlaps(const spiral_tensor* t, const spiral_tensor* b) {
+  const auto extent = [](const spiral_tensor* u) {
+    size_t end = elem_size(u->type) * static_cast<size_t>(u->ne[0]);
+    for (int d = 1; d < SPIRAL_MAX_DIMS; ++d) end += static_cast<size_t>(u->ne[d] - 1) * u->nb[d];
+    return end;
+  };
+  const uintptr_t p = reinterpret_cast<uintptr_t>(t->data), q = reinterpret_cast<uintptr_t>(b->data);
+  return p < q + extent(b) && q < p + extent(t);
 }
 
 int grow_scratch(spiral_backend* be, size_t need) {
@@ -733,23 +758,42 @@ int spiral_backend_graph_compute(spiral_backend* be, const spiral_cgraph* graph)
   DeviceGuard g(be->device);
   int rc = grow_scratch(be, need);
   if (rc != SPIRAL_OK) return rc;
+  const spiral_tensor* held = nullptr;  // see compute_mul_mat
   for (int32_t i = 0; i < graph->n_nodes && rc == SPIRAL_OK; ++i) {
     const spiral_tensor* t = graph->nodes[i];
     if (fusable_glu(graph, i)) {
       rc = compute_mul_mat_id_glu(be, t, graph->nodes[i + 1]);
+      held = nullptr;
       ++i;
       continue;
     }
     if (fusable_glu_split(graph, i)) {
       rc = compute_mul_mat_id_glu_split(be, graph->nodes[i + 2]);
+      held = nullptr;
       i += 2;
       continue;
     }
     switch (t->op) {
-      case SPIRAL_OP_MUL_MAT: rc = compute_mul_mat(be, t); break;
-      case SPIRAL_OP_GET_ROWS: rc = compute_get_rows(be, t); break;
-      case SPIRAL_OP_MUL_MAT_ID: rc = compute_mul_mat_id(be, t); break;
-      case SPIRAL_OP_GLU: rc = compute_glu(be, t); break;
+      case SPIRAL_OP_MUL_MAT:
+        rc = compute_mul_mat(be, t, held);
+        if (held != nullptr && overlaps(t, held)) held = nullptr;
+        break;
+      case SPIRAL_OP_GET_ROWS: {
+        uint16_t* copy = copy_for_next(be, graph, i);
+        rc = compute_get_rows(be, t, copy);
+        held = copy != nullptr ? t : nullptr;
+        break;
+      }
+      case SPIRAL_OP_MUL_MAT_ID:
+        rc = compute_mul_mat_id(be, t);
+        held = nullptr;
+        break;
+      case SPIRAL_OP_GLU: {
+        uint16_t* copy = copy_for_next(be, graph, i);
+        rc = compute_glu(be, t, copy);
+        held = copy != nullptr ? t : nullptr;
+        break;
+      }
       default: break;  // views and no-ops
     }
   }

@@ -280,4 +280,14 @@ int allow_dynamic_lds(const void* kernel, int bytes);
 int dequant_rows(int type, const void* w, int64_t n_rows, int64_t k, int64_t row0, int64_t rows, uint16_t* out,
                  int64_t ld_out, hipStream_t s);
 
+// spiral_get_rows that also leaves the F32 rows as contiguous bf16 in `copy`
+// (dequant.hip), and the GLU forms that do the same (api.hip); copy may be null.
+int get_rows_copy(int type, const void* w, int64_t n_rows, int64_t k, const int32_t* ids, int64_t n_ids, void* out,
+                  int out_type, int64_t ld_out, uint16_t* copy, void* stream);
+int glu_entry(int glu_op, int swapped, float alpha, float limit, const float* x, int64_t ldx, int64_t F, int64_t rows,
+              float* y, int64_t ldy, uint16_t* copy, void* stream);
+int glu_split_entry(int glu_op, int swapped, float alpha, float limit, const float* gate, int64_t ldg,
+                    const float* up, int64_t ldu, int64_t F, int64_t rows, float* y, int64_t ldy, uint16_t* copy,
+                    void* stream);
+
 }  // namespace spiral

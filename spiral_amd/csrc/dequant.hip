@@ -55,7 +55,7 @@ template <int TYPE, bool F32_OUT>
 __global__ void __launch_bounds__(256) get_rows_kernel(const uint8_t* __restrict__ w, int64_t n_rows,
                                                        int64_t nb, uint32_t groups_per_row, uint32_t wg_per_row,
                                                        const int32_t* __restrict__ ids, void* __restrict__ out,
-                                                       int64_t ld_out) {
+                                                       int64_t ld_out, uint16_t* __restrict__ copy) {
   const uint32_t r = blockIdx.x / wg_per_row;
   const uint32_t g = (blockIdx.x - r * wg_per_row) * 256 + threadIdx.x;
   if (g >= groups_per_row) return;
@@ -77,6 +77,8 @@ __global__ void __launch_bounds__(256) get_rows_kernel(const uint8_t* __restrict
     float* p = static_cast<float*>(out) + r * ld_out + 8 * g;
     store_stream16(p, make_uint4(o.x << 16, o.x & 0xffff0000u, o.y << 16, o.y & 0xffff0000u));
     store_stream16(p + 4, make_uint4(o.z << 16, o.z & 0xffff0000u, o.w << 16, o.w & 0xffff0000u));
+    // the same rows as bf16, back to back, for the product that reads them next
+    if (copy != nullptr) *reinterpret_cast<uint4*>(copy + (static_cast<int64_t>(r) * groups_per_row + g) * 8) = o;
   } else {
     store_stream16(static_cast<uint16_t*>(out) + r * ld_out + 8 * g, o);
   }
@@ -108,25 +110,10 @@ int dequant_rows(int type, const void* w, int64_t n_rows, int64_t k, int64_t row
   return launch_status();
 }
 
-}  // namespace spiral
-
-using namespace spiral;
-
-extern "C" {
-
-int spiral_dequant_bf16(int type, const void* w, int64_t n_rows, int64_t k, uint16_t* out,
-                        int64_t ld_out, void* stream) {
-  if (!is_quant_type(type)) return SPIRAL_ERR_TYPE;
-  if (w == nullptr || out == nullptr) return SPIRAL_ERR_NULL;
-  if (n_rows <= 0 || k <= 0 || k % block_elems(type) != 0 || ld_out < k) return SPIRAL_ERR_SHAPE;
-  if (!aligned16(w) || !aligned16(out) || ld_out % 8 != 0) return SPIRAL_ERR_ALIGN;
-  int rc = require_device();
-  if (rc != SPIRAL_OK) return rc;
-  return dequant_rows(type, w, n_rows, k, 0, n_rows, out, ld_out, static_cast<hipStream_t>(stream));
-}
-
-int spiral_get_rows(int type, const void* w, int64_t n_rows, int64_t k, const int32_t* ids,
-                    int64_t n_ids, void* out, int out_type, int64_t ld_out, void* stream) {
+// spiral_get_rows; with F32 output and `copy` set, also writes the rows there
+// as contiguous bf16 (16-byte aligned).
+int get_rows_copy(int type, const void* w, int64_t n_rows, int64_t k, const int32_t* ids, int64_t n_ids, void* out,
+                  int out_type, int64_t ld_out, uint16_t* copy, void* stream) {
   if (!is_quant_type(type)) return SPIRAL_ERR_TYPE;
   if (out_type != SPIRAL_TYPE_BF16 && out_type != SPIRAL_TYPE_F32) return SPIRAL_ERR_TYPE;
   if (n_ids == 0) return SPIRAL_OK;
@@ -146,10 +133,10 @@ int spiral_get_rows(int type, const void* w, int64_t n_rows, int64_t k, const in
   do {                                                                                          \
     if (out_type == SPIRAL_TYPE_F32)                                                            \
       hipLaunchKernelGGL((get_rows_kernel<T, true>), grid, dim3(256), 0, s, W, n_rows, nb, g32, \
-                         w32, ids, out, ld_out);                                                \
+                         w32, ids, out, ld_out, copy);                                                \
     else                                                                                        \
       hipLaunchKernelGGL((get_rows_kernel<T, false>), grid, dim3(256), 0, s, W, n_rows, nb,     \
-                         g32, w32, ids, out, ld_out);                                           \
+                         g32, w32, ids, out, ld_out, copy);                                           \
   } while (0)
   switch (type) {
     case SPIRAL_TYPE_Q4_0: SPIRAL_GET_ROWS(SPIRAL_TYPE_Q4_0); break;
@@ -162,6 +149,28 @@ int spiral_get_rows(int type, const void* w, int64_t n_rows, int64_t k, const in
   }
 #undef SPIRAL_GET_ROWS
   return launch_status();
+}
+
+}  // namespace spiral
+
+using namespace spiral;
+
+extern "C" {
+
+int spiral_dequant_bf16(int type, const void* w, int64_t n_rows, int64_t k, uint16_t* out,
+                        int64_t ld_out, void* stream) {
+  if (!is_quant_type(type)) return SPIRAL_ERR_TYPE;
+  if (w == nullptr || out == nullptr) return SPIRAL_ERR_NULL;
+  if (n_rows <= 0 || k <= 0 || k % block_elems(type) != 0 || ld_out < k) return SPIRAL_ERR_SHAPE;
+  if (!aligned16(w) || !aligned16(out) || ld_out % 8 != 0) return SPIRAL_ERR_ALIGN;
+  int rc = require_device();
+  if (rc != SPIRAL_OK) return rc;
+  return dequant_rows(type, w, n_rows, k, 0, n_rows, out, ld_out, static_cast<hipStream_t>(stream));
+}
+
+int spiral_get_rows(int type, const void* w, int64_t n_rows, int64_t k, const int32_t* ids,
+                    int64_t n_ids, void* out, int out_type, int64_t ld_out, void* stream) {
+  return get_rows_copy(type, w, n_rows, k, ids, n_ids, out, out_type, ld_out, nullptr, stream);
 }
 
 }  // extern "C"

@@ -672,18 +672,21 @@ __device__ __forceinline__ float glu_pair(int op, float a, float b, float alpha,
   return glu_act(op, a) * b;
 }
 
+// `copy` (may be null): y as bf16 too, rows of n back to back.
 // Standalone ggml GLU over rows of 2n floats: y[r][i] = act(h0[i]) * h1[i]
 // with (h0, h1) = (x[r][0 .. n), x[r][n .. 2n)), swapped: the other order.
 __global__ void __launch_bounds__(256) glu_kernel(const float* __restrict__ x, int64_t ldx, float* __restrict__ y,
                                                   int64_t ldy, int64_t n, int64_t rows, int op, int swapped,
-                                                  float alpha, float limit) {
+                                                  float alpha, float limit, uint16_t* __restrict__ copy) {
   const int64_t total = n * rows;
   for (int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; i < total;
        i += static_cast<int64_t>(gridDim.x) * 256) {
     const int64_t r = i / n, c = i - r * n;
     const float* xr = x + r * ldx;
     const float a = xr[swapped ? c + n : c], b = xr[swapped ? c : c + n];
-    y[r * ldy + c] = glu_pair(op, a, b, alpha, limit);
+    const float v = glu_pair(op, a, b, alpha, limit);
+    y[r * ldy + c] = v;
+    if (copy != nullptr) copy[i] = __builtin_bit_cast(uint16_t, static_cast<__bf16>(v));
   }
 }
 
@@ -692,13 +695,16 @@ __global__ void __launch_bounds__(256) glu_kernel(const float* __restrict__ x, i
 __global__ void __launch_bounds__(256) glu_split_kernel(const float* __restrict__ xg, int64_t ldg,
                                                         const float* __restrict__ xu, int64_t ldu,
                                                         float* __restrict__ y, int64_t ldy, int64_t n, int64_t rows,
-                                                        int op, int swapped, float alpha, float limit) {
+                                                        int op, int swapped, float alpha, float limit,
+                                                        uint16_t* __restrict__ copy) {
   const int64_t total = n * rows;
   for (int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; i < total;
        i += static_cast<int64_t>(gridDim.x) * 256) {
     const int64_t r = i / n, c = i - r * n;
     const float g = xg[r * ldg + c], u = xu[r * ldu + c];
-    y[r * ldy + c] = swapped ? glu_pair(op, u, g, alpha, limit) : glu_pair(op, g, u, alpha, limit);
+    const float v = swapped ? glu_pair(op, u, g, alpha, limit) : glu_pair(op, g, u, alpha, limit);
+    y[r * ldy + c] = v;
+    if (copy != nullptr) copy[i] = __builtin_bit_cast(uint16_t, static_cast<__bf16>(v));
   }
 }
 
@@ -1608,23 +1614,23 @@ int moe(int type, const void* w, int64_t expert_stride, int64_t n_expert, int64_
 // Standalone GLU over `rows` rows of 2n floats; arguments validated by the
 // caller.
 int glu(int op, int swapped, const float* x, int64_t ldx, int64_t n, int64_t rows, float* y, int64_t ldy,
-        hipStream_t s, float alpha, float limit) {
+        hipStream_t s, float alpha, float limit, uint16_t* copy) {
   const int64_t total = n * rows;
   if (total == 0) return SPIRAL_OK;
   const int64_t blocks = std::min<int64_t>(ceil_div(total, 256), 8 * static_cast<int64_t>(device_cu_count()));
   hipLaunchKernelGGL(glu_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s, x, ldx, y, ldy, n, rows, op,
-                     swapped, alpha, limit);
+                     swapped, alpha, limit, copy);
   return launch_status();
 }
 
 // Split form: gate rows at xg (stride ldg), up rows at xu (stride ldu).
 int glu_split(int op, int swapped, const float* xg, int64_t ldg, const float* xu, int64_t ldu, int64_t n,
-              int64_t rows, float* y, int64_t ldy, hipStream_t s, float alpha, float limit) {
+              int64_t rows, float* y, int64_t ldy, hipStream_t s, float alpha, float limit, uint16_t* copy) {
   const int64_t total = n * rows;
   if (total == 0) return SPIRAL_OK;
   const int64_t blocks = std::min<int64_t>(ceil_div(total, 256), 8 * static_cast<int64_t>(device_cu_count()));
   hipLaunchKernelGGL(glu_split_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s, xg, ldg, xu, ldu, y, ldy,
-                     n, rows, op, swapped, alpha, limit);
+                     n, rows, op, swapped, alpha, limit, copy);
   return launch_status();
 }
 
