@@ -53,9 +53,15 @@
 
 #include "common.h"
 #include "dequant_impl.h"
+#include "glu.h"
 #include "moe_piece.h"
 
 namespace spiral {
+bool moe_tile_fits(int type, int64_t n_expert, int64_t k, int64_t x_slots, int64_t n_pairs, int64_t top_k);
+int moe_tile(int type, const void* w, const void* w_up, int64_t expert_stride, int64_t n_expert, int64_t n_rows,
+             int64_t k, const uint16_t* x, int64_t x_slots, int64_t n_pairs, int64_t top_k, const int32_t* offsets,
+             const int32_t* list, void* y, bool f32, int glu_op, int swapped, hipStream_t s);
+
 namespace {
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
@@ -643,22 +649,6 @@ __global__ void __launch_bounds__(256) moe_kernel(const uint8_t* __restrict__ w,
 
 
 // ---- GLU activations (ggml GLU ops, fp32) -----------------------------------
-// act(a) * b for the ggml GLU variants (ids as in include/spiral_ggml.h):
-// REGLU relu, GEGLU gelu (tanh form), SWIGLU silu, GEGLU_ERF gelu (erf form),
-// GEGLU_QUICK x * sigmoid(1.702 x).
-__device__ __forceinline__ float glu_act(int op, float a) {
-  switch (op) {
-    case SPIRAL_GLU_REGLU: return a > 0.0f ? a : 0.0f;
-    case SPIRAL_GLU_GEGLU: {
-      const float u = 0.7978845608028654f * a * (1.0f + 0.044715f * a * a);  // sqrt(2/pi) (a + 0.044715 a^3)
-      return 0.5f * a * (1.0f + tanhf(u));
-    }
-    case SPIRAL_GLU_SWIGLU: return a / (1.0f + expf(-a));
-    case SPIRAL_GLU_GEGLU_ERF: return 0.5f * a * (1.0f + erff(a * 0.7071067811865476f));
-    default: return a / (1.0f + expf(-1.702f * a));  // SPIRAL_GLU_GEGLU_QUICK
-  }
-}
-
 // One output of a standalone GLU: act(a) * b, a the activated half. SWIGLU_OAI
 // (gpt-oss, as ggml computes it): with x = min(a, limit) and
 // y = clamp(b, -limit, limit), x / (1 + exp(-alpha x)) * (y + 1); min and
@@ -1561,13 +1551,17 @@ int moe(int type, const void* w, int64_t expert_stride, int64_t n_expert, int64_
   if (glu && !stream_ok) return SPIRAL_ERR_SHAPE;
   int32_t* offsets = nullptr;
   int32_t* list = nullptr;
-  if (n_pairs > kFusedPairs) {
+  const bool tiled = moe_tile_fits(type, n_expert, k, x_slots, n_pairs, top_k);
+  if (n_pairs > kFusedPairs || tiled) {
     offsets = static_cast<int32_t*>(workspace);
     list = offsets + n_expert + 1;
     hipLaunchKernelGGL(route_kernel, dim3(1), dim3(kRouteThreads), 0, s, ids, static_cast<int32_t>(n_pairs),
                        static_cast<int32_t>(n_expert), offsets, list, y, glu ? n_rows / 2 : n_rows, f32);
     if (hipGetLastError() != hipSuccess) return SPIRAL_ERR_HIP;
   }
+  if (tiled)
+    return moe_tile(type, w, w_up, expert_stride, n_expert, n_rows, k, x, x_slots, n_pairs, top_k, offsets, list, y,
+                    f32 != 0, glu_op, swapped, s);
   if (stream_ok) {
 #define SPIRAL_MOE_STREAM_AS(T, F, G) \
   launch_stream<T, F, G>(w, expert_stride, n_expert, n_rows, k, x, x_slots, ids, n_pairs, top_k, offsets, list, y, \

@@ -1,0 +1,93 @@
+"""GPU parity of MUL_MAT_ID's tiled form (spiral_amd/csrc/moe_tile.hip), which
+takes batches of more than 16 routed tokens an expert: every format it has, rows
+that are no multiple of its 96 (48 features with GLU), of 16 or of 4, one to five
+super-blocks of k, experts of no tokens, of one, and of counts at the edges of
+its token tiles (32, 64, 80 and over), per-slot inputs, ids routed nowhere, the
+fused GLU form merged and split. Equal bit for bit to the same tokens in small
+calls (the streaming form), and to the oracle within the product bars.
+"""
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import oracle as O
+from spiral_amd import ops
+from test_gpu_parity import _moe_inputs, _moe_ref, check_moe, dev_bf16
+
+pytestmark = pytest.mark.gpu
+
+FORMATS = [O.Q4_0, O.Q4_K, O.Q5_K, O.IQ4_NL]
+
+
+def ids_of(counts):
+    """[tokens, 1] ids giving expert e counts[e] tokens, shuffled; the last
+    entry counts the tokens routed nowhere."""
+    ids = np.concatenate([np.full(c, e if e + 1 < len(counts) else -1) for e, c in enumerate(counts)])
+    return np.random.default_rng(1).permutation(ids).astype(np.int32)[:, None]
+
+
+def small_calls(call, x, ids, step):
+    return torch.cat([call(x[t:t + step].contiguous(), ids[t:t + step].contiguous())
+                      for t in range(0, ids.shape[0], step)])
+
+
+@pytest.mark.parametrize("out_dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n,k", [(96, 256), (100, 768), (198, 1280), (8, 512)])
+@pytest.mark.parametrize("qtype", FORMATS)
+def test_tile(cuda, qtype, n, k, out_dtype):
+    ids = ids_of([32, 1, 0, 64, 81, 7])  # 178 pairs routed to 5 experts
+    e, tokens = 5, ids.shape[0]
+    w, per, raws, ids, x = _moe_inputs(cuda, qtype, e, n, k, tokens, 1, 1, 400, ids)
+    xd, idd = dev_bf16(x, cuda), torch.from_numpy(ids).to(cuda)
+
+    def call(xs, i):
+        return ops.mul_mat_id(qtype, w, per, e, n, k, xs, i, out_dtype=out_dtype)
+
+    y = call(xd, idd)
+    assert torch.equal(y, small_calls(call, xd, idd, 10))
+    got = y.float().cpu().numpy()
+    assert not got[ids < 0].any()
+    check_moe(got, _moe_ref(qtype, raws, n, k, ids, x), out_dtype == torch.float32)
+
+
+@pytest.mark.parametrize("split", [False, True])
+@pytest.mark.parametrize("F,k", [(48, 256), (50, 768), (132, 1024)])
+@pytest.mark.parametrize("qtype", FORMATS)
+def test_tile_glu(cuda, qtype, F, k, split):
+    """Merged: equal to the product and the standalone GLU. Split: the same
+    stacks' halves as two matrices; two tokens slots an expert pair."""
+    e, tokens, top = 4, 160, 2
+    n = 2 * F
+    w, per, raws, ids, x = _moe_inputs(cuda, qtype, e, n, k, tokens, top, 1, 410)
+    xd, idd = dev_bf16(x, cuda), torch.from_numpy(ids).to(cuda)
+    prod = ops.mul_mat_id(qtype, w, per, e, n, k, xd, idd, out_dtype=torch.float32)
+    want = ops.glu(prod, ops.GLU_SWIGLU)
+    if not split:
+        got = ops.mul_mat_id_glu(qtype, w, per, e, n, k, xd, idd, ops.GLU_SWIGLU, out_dtype=torch.float32)
+    else:
+        half = [torch.stack([ops.to_planar(qtype, torch.from_numpy(np.ascontiguousarray(
+            r.reshape(n, -1)[i * F:(i + 1) * F]).reshape(-1)).to(cuda), F, k) for r in raws]) for i in range(2)]
+        got = ops.mul_mat_id_glu_split(qtype, half[0], half[1], half[0].shape[1], e, F, k, xd, idd, ops.GLU_SWIGLU,
+                                       out_dtype=torch.float32)
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("qtype", FORMATS)
+def test_tile_slots_and_many_tiles(cuda, qtype):
+    """Per-slot inputs and an expert of several tiles; a base address of y that
+    is only 4-byte aligned."""
+    e, n, k, tokens, top = 3, 70, 512, 300, 2
+    w, per, raws, ids, x = _moe_inputs(cuda, qtype, e, n, k, tokens, top, top, 420)
+    xd, idd = dev_bf16(x, cuda), torch.from_numpy(ids).to(cuda)
+
+    def call(xs, i):
+        flat = torch.full((i.shape[0] * top * n + 1,), 7.0, dtype=torch.float32, device=cuda)
+        ops.mul_mat_id(qtype, w, per, e, n, k, xs, i, out=flat[1:].view(i.shape[0], top, n))
+        assert flat[0] == 7.0
+        return flat[1:].view(i.shape[0], top, n)
+
+    y = call(xd, idd)
+    assert torch.equal(y, small_calls(call, xd, idd, 10))
+    check_moe(y.cpu().numpy(), _moe_ref(qtype, raws, n, k, ids, x), True)
