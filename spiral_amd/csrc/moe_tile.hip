@@ -54,7 +54,10 @@ constexpr uint32_t kNone = 0x80000000u;  // past every buffer: fetches nothing
 template <int TYPE>
 constexpr bool kHighBits = TYPE == SPIRAL_TYPE_Q5_K;
 template <int TYPE>
-constexpr bool kSplitX = TYPE == SPIRAL_TYPE_Q4_0 || TYPE == SPIRAL_TYPE_IQ4_NL;
+constexpr bool kSplitX = TYPE == SPIRAL_TYPE_Q4_0 || is_iq4(TYPE);
+// Bytes of a row's scale entry for 256 k.
+template <int TYPE>
+constexpr int kEntry = TYPE == SPIRAL_TYPE_IQ4_XS ? 8 : 16;
 
 // LDS: x stages, code stages, scale-entry stages, [high-bit stages], decoded scales.
 constexpr int kXStage = kTokens * 256, kQStage = kRows * 128, kMStage = kRows * 16, kHStage = kRows * 32;
@@ -66,8 +69,8 @@ struct Lds {
 };
 static_assert(Lds<SPIRAL_TYPE_Q5_K>::kBytes <= 80 * 1024, "two workgroups a CU");
 
-// (scale, offset) of 32-weight group j of a row from its 16-byte entry: Q4_0 and
-// IQ4_NL eight fp16 d, the K-quants d, dmin and the packed scales.
+// (scale, offset) of 32-weight group j of a row from its entry: Q4_0 and IQ4_NL
+// eight fp16 d, the K-quants d, dmin and the packed scales, IQ4_XS d and its own.
 template <int TYPE>
 __device__ __forceinline__ f32x2_t decode_scale(const uint8_t* entry, int j) {
   if constexpr (is_kquant(TYPE)) {
@@ -75,6 +78,10 @@ __device__ __forceinline__ f32x2_t decode_scale(const uint8_t* entry, int j) {
     const uint32_t sm = kq_chunk_scales(m.y, m.z, m.w, static_cast<uint32_t>(j) >> 1) >> (16 * (j & 1));
     return f32x2_t{fp16_ieee(m.x & 0xffffu) * 16777216.0f * static_cast<float>(sm & 0xffu),
                        -(fp16_ieee(m.x >> 16) * static_cast<float>((sm >> 8) & 0xffu))};
+  } else if constexpr (TYPE == SPIRAL_TYPE_IQ4_XS) {
+    const u32x2_t m = *reinterpret_cast<const u32x2_t*>(entry);
+    const float sc = iq4xs_scale(make_uint2(m.x, m.y), j);
+    return f32x2_t{sc, -1152.0f * sc};
   } else {
     const uint32_t d = reinterpret_cast<const uint16_t*>(entry)[j];
     const float m = TYPE == SPIRAL_TYPE_Q4_0 ? fp16_scale(d) : fp16_ieee(d);
@@ -120,7 +127,7 @@ __global__ void __launch_bounds__(kThreads, 2)
     Matrix M;
     M.q = buffer_rsrc(p, codes);
     M.h = kHighBits<TYPE> ? buffer_rsrc(p + codes, hbytes) : M.q;
-    M.m = buffer_rsrc(p + codes + hbytes, mat_rows * nsb * 16);
+    M.m = buffer_rsrc(p + codes + hbytes, mat_rows * nsb * kEntry<TYPE>);
     return M;
   };
   const bool split = GLU && w_up != nullptr;
@@ -139,14 +146,21 @@ __global__ void __launch_bounds__(kThreads, 2)
     const uint32_t lr = 24 * s + 8 * i + (lane >> 3);
     qoff[i] = row_of(lr) * (nsb * 128) + (((lane & 7u) ^ ((lr >> 1) & 7u)) * 16);
   }
-  const uint32_t moff = row_of(24 * s + min(lane, 23u)) * (nsb * 16);
+  // (IQ4_XS's 8-byte entries go a dword a lane)
+  constexpr uint32_t kMLane = kEntry<TYPE> == 8 ? 2 : 1;
+  const uint32_t moff = row_of(24 * s + min(lane / kMLane, 23u)) * (nsb * kEntry<TYPE>) + (lane % kMLane) * 4;
   const uint32_t hoff = kHighBits<TYPE> ? row_of(24 * s + min(lane >> 1, 23u)) * (nsb * 32) + (lane & 1u) * 16 : 0;
   const auto load_w = [&](uint32_t sb) {
     const uint32_t st = sb & 1u;
     const Matrix& M = s < 2 ? lo : hi;
 #pragma unroll
     for (int i = 0; i < 3; ++i) dma16(M.q, smem + L::kQ + st * kQStage + (24 * s + 8 * i) * 128, qoff[i], sb * 128);
-    if (lane < 24) dma16(M.m, smem + L::kM + st * kMStage + 24 * s * 16, moff, sb * 16);
+    uint8_t* entries = smem + L::kM + st * kMStage + 24 * s * kEntry<TYPE>;
+    if constexpr (kEntry<TYPE> == 8) {
+      if (lane < 48) dma4(M.m, entries, moff, sb * 8);
+    } else {
+      if (lane < 24) dma16(M.m, entries, moff, sb * 16);
+    }
     if constexpr (kHighBits<TYPE>) {
       if (lane < 48) dma16(M.h, smem + L::kH + st * kHStage + 24 * s * 32, hoff, sb * 32);
     }
@@ -209,7 +223,7 @@ __global__ void __launch_bounds__(kThreads, 2)
         for (int i = 0; i < kRows * 8 / kThreads; ++i) {
           const uint32_t n = tid + kThreads * i, lr = n >> 3, j = n & 7u;
           *reinterpret_cast<f32x2_t*>(smem + L::kS + lr * 64 + ((j ^ (2 * ((lr >> 2) & 3u))) * 8)) =
-              decode_scale<TYPE>(smem + L::kM + (sb & 1u) * kMStage + lr * 16, static_cast<int>(j));
+              decode_scale<TYPE>(smem + L::kM + (sb & 1u) * kMStage + lr * kEntry<TYPE>, static_cast<int>(j));
         }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
@@ -357,17 +371,18 @@ int launch_tile(const void* w, const void* w_up, int64_t expert_stride, int64_t 
 
 }  // namespace
 
-// Whether the tiled form takes this MUL_MAT_ID: formats of 16-byte scale entries
-// a 256 k, 32-bit offsets, and enough tokens an expert. The streaming form takes
-// 16 tokens a pass up to there, and reads weights ahead better: gate_up and down
-// of 128 experts, 2048 / 768, Q4_K, us, streaming against this form at 10, 16 and
-// 24 tokens an expert: 146 and 163, 196 and 166, 236 and 174 (Q4_0 130 and 157,
-// 160 and 161, 199 and 171). Past k = 2304 its passes stay at 16 tokens: 60
-// experts, 3072 / 1536, 12 tokens: 268 and 195 (Q4_0 241 and 188).
+// Whether the tiled form takes this MUL_MAT_ID: formats of 4-bit codes (and Q5_K),
+// 32-bit offsets, and enough tokens an expert. Below that the streaming form reads
+// its weights ahead better: gate_up and down of 128 experts, 2048 / 768, us,
+// streaming against this form at 17, 20 and 24 tokens an expert (its passes take
+// 32): Q4_K 142 and 166, 145 and 167, 237 and 176; Q4_0 123 and 160, 162 and 164,
+// 199 and 173; IQ4_XS 159 and 189, 210 and 185, 267 and 194. Past k = 2304 its
+// passes stay at 16: 60 experts, 3072 / 1536, 13 tokens: Q4_K 310 and 221, Q4_0
+// 246 and 203, IQ4_XS 264 and 239.
 bool moe_tile_fits(int type, int64_t n_expert, int64_t k, int64_t x_slots, int64_t n_pairs, int64_t top_k) {
-  if (type != SPIRAL_TYPE_Q4_0 && type != SPIRAL_TYPE_IQ4_NL && !is_kquant(type)) return false;
+  if (type != SPIRAL_TYPE_Q4_0 && !is_iq4(type) && !is_kquant(type)) return false;
   if (k % 256 != 0 || n_expert > 65535 || n_pairs / top_k * x_slots * k * 2 >= (int64_t(1) << 31)) return false;
-  return n_pairs > (k > 2304 ? 12 : 16) * n_expert;
+  return n_pairs >= (k > 2304 ? 13 : 24) * n_expert;
 }
 
 // Arguments validated by the caller (moe); offsets and list from the route kernel.
@@ -386,6 +401,7 @@ int moe_tile(int type, const void* w, const void* w_up, int64_t expert_stride, i
     SPIRAL_TILE(SPIRAL_TYPE_Q4_K);
     SPIRAL_TILE(SPIRAL_TYPE_Q5_K);
     SPIRAL_TILE(SPIRAL_TYPE_IQ4_NL);
+    SPIRAL_TILE(SPIRAL_TYPE_IQ4_XS);
     default: return SPIRAL_ERR_TYPE;
   }
 #undef SPIRAL_TILE

@@ -1,5 +1,6 @@
 """GPU parity of MUL_MAT_ID's tiled form (spiral_amd/csrc/moe_tile.hip), which
-takes batches of more than 16 routed tokens an expert: every format it has, rows
+takes batches of 24 routed tokens an expert or more (13 past k = 2304): every
+format it has, rows
 that are no multiple of its 96 (48 features with GLU), of 16 or of 4, one to five
 super-blocks of k, experts of no tokens, of one, and of counts at the edges of
 its token tiles (32, 64, 80 and over), per-slot inputs, ids routed nowhere, the
@@ -17,7 +18,7 @@ from test_gpu_parity import _moe_inputs, _moe_ref, check_moe, dev_bf16
 
 pytestmark = pytest.mark.gpu
 
-FORMATS = [O.Q4_0, O.Q4_K, O.Q5_K, O.IQ4_NL]
+FORMATS = [O.Q4_0, O.Q4_K, O.Q5_K, O.IQ4_NL, O.IQ4_XS]
 
 
 def ids_of(counts):
