@@ -6,20 +6,22 @@ synchronizing. Weight tensors are uint8 device tensors in the library's
 planar layout (see to_planar); bf16 data is carried in torch.bfloat16 tensors.
 """
 
-import ctypes
-
 import torch
 
 from ._lib import TYPE_BF16, TYPE_F32, check, lib
 from . import BLOCK_ELEMS, row_bytes
 
 
+# Pointers and streams are passed as plain integers (the functions' argtypes make
+# them void pointers), and the stream is read without building a torch Stream
+# object: both show at the smallest calls, which the host issues slower than the
+# GPU runs them.
 def _stream():
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def _ptr(t):
-    return ctypes.c_void_p(t.data_ptr())
+    return t.data_ptr()
 
 
 def _out_type(dtype):
