@@ -270,14 +270,19 @@ int compute_mul_mat(spiral_backend* be, const spiral_tensor* t, const spiral_ten
   int rc = SPIRAL_OK;
   int64_t ld1 = b->ne[0], ld2 = ld1 * b->ne[1], ld3 = ld2 * b->ne[2];
   const uint16_t* xb = reinterpret_cast<const uint16_t*>(be->scratch);
+  // The workspace lies behind the activation's copy. Rows read in place have
+  // none, so there it is the start of the scratch, where a held copy lies.
+  uint8_t* ws = be->scratch + act_scratch(b);
+  const int64_t wsb = static_cast<int64_t>(mul_mat_workspace(t));
   if (held != b) {
     xb = act_bf16(b, be->scratch, false, be->stream, ld1, ld2, ld3, rc);
     if (rc != SPIRAL_OK) return rc;
-    if (act_scratch(b) != 0) held = b;
+    if (act_scratch(b) != 0)
+      held = b;
+    else if (wsb > 0)
+      held = nullptr;
   }
   const int64_t r2 = b->ne[2] / a->ne[2], r3 = b->ne[3] / a->ne[3];
-  uint8_t* ws = be->scratch + act_scratch(b);
-  const int64_t wsb = static_cast<int64_t>(mul_mat_workspace(t));
   for (int64_t i3 = 0; i3 < b->ne[3]; ++i3) {
     for (int64_t i2 = 0; i2 < b->ne[2]; ++i2) {
       const uint8_t* w = static_cast<const uint8_t*>(a->data) + (i2 / r2) * a->nb[2] + (i3 / r3) * a->nb[3];

@@ -3,7 +3,8 @@ for bit: get_rows and GLU leave a bf16 copy of their rows for the product behind
 them, and products over one activation share its conversion
 (spiral_amd/csrc/backend.hip). Covered: one row (GEMV), a few (small batch) and
 many (GEMM); both GLU forms; batched rows; an activation that a product
-overwrites; products that read something else than the node before them.
+overwrites; products that read something else than the node before them; a
+product between them whose workspace takes the place of their copy.
 """
 
 import numpy as np
@@ -118,5 +119,35 @@ def test_batched_rows(cuda):
     ids.data = dev.data_ptr()
     x = ggml.get_rows(t, ids)
     nodes = [x, ggml.mul_mat(w, x)]
+    whole, single = whole_and_single(nodes, place(nodes))
+    assert all(torch.equal(a, b) and not (a == 7.0).any() for a, b in zip(whole, single))
+
+
+# A bf16 activation is read in place, so its product's workspace starts where the
+# copy lies: the packed rows, the sums of two k ranges, the dequantized matrix;
+# and a product of few rows, which takes no workspace.
+@pytest.mark.parametrize("qtype,m,n,k", [(O.Q6_K, 40, 96, 512), (O.Q4_0, 17, 300, 4096 + 96),
+                                         (O.Q4_0, 257, 7001, 64), (O.Q4_K, 5, 96, 512)])
+@pytest.mark.parametrize("made", [False, True])
+def test_bf16_product_between(cuda, qtype, m, n, k, made):
+    """x, a bf16 activation's product, x again, with x given (converted by its
+    first product) and made by get_rows (which leaves the copy)."""
+    h, w_rows = 256, 64
+    buf = ggml.Buffer(8 << 20)
+    w0, w2 = quant(buf, O.Q4_K, w_rows, h, 1), quant(buf, O.Q4_K, w_rows, h, 2)
+    w1 = quant(buf, qtype, n, k, 3)
+    z_mem = torch.randn((m, k), device="cuda").to(torch.bfloat16)
+    z = ggml.new_tensor(ggml.TYPE_BF16, (k, m))
+    z.data = z_mem.data_ptr()
+    if made:
+        ids, keep = ids_tensor([(7 * i) % w_rows for i in range(40)])
+        x = ggml.get_rows(w0, ids)
+    else:
+        x_mem = torch.randn((40, h), device="cuda")
+        x = ggml.new_tensor(ggml.TYPE_F32, (h, 40))
+        x.data = x_mem.data_ptr()
+    nodes = [ggml.mul_mat(w0, x), ggml.mul_mat(w1, z), ggml.mul_mat(w2, x)]
+    if made:
+        nodes.insert(0, x)
     whole, single = whole_and_single(nodes, place(nodes))
     assert all(torch.equal(a, b) and not (a == 7.0).any() for a, b in zip(whole, single))
