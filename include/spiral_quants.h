@@ -192,7 +192,11 @@ int spiral_get_rows(int type, const void* w, int64_t n_rows, int64_t k,
  * case workspace may be NULL); from a few hundred rows, where that is
  * faster, it dequantizes the matrix into `workspace` once instead (up to
  * 256 MiB at a time), and long rows that leave CUs idle are multiplied in
- * ranges of k whose F32 sums go through `workspace`. A workspace of only the
+ * ranges of k whose F32 sums go through `workspace`. Dequantized once, a bf16
+ * result is one chain of fp32 additions over k (k / 32 of them) where the other
+ * forms have shorter ones: at k = 14336 its error before rounding is 7e-7 of the
+ * outputs' root mean square against 3.4e-7, its error after it the same 1.66e-3;
+ * F32 results keep short chains. A workspace of only the
  * rewritten x (m rounded up to 16, times k, 2 bytes each) is accepted too
  * and runs without either. A workspace must not be shared by calls in
  * flight at the same time. The small-batch form needs y within 2 GiB

@@ -94,7 +94,8 @@ __device__ __forceinline__ void interleave() {
 template <int MF, int NF, bool F32_OUT>
 __global__ void __launch_bounds__(kThreads, 2)
     dense_kernel(const uint16_t* __restrict__ x, uint32_t ldx, uint32_t m, const uint16_t* __restrict__ wb, uint32_t n,
-                 uint32_t k, void* __restrict__ y, int64_t ldy, uint32_t tiles_m, uint32_t tiles_n) {
+                 uint32_t k, void* __restrict__ y, int64_t ldy, uint32_t tiles_m, uint32_t tiles_n,
+                 uint32_t flush_steps) {
   constexpr int BM = 64 * MF, BN = 32 * NF;
   using S = Stages<MF, NF>;
   extern __shared__ __align__(1024) uint8_t smem[];
@@ -176,11 +177,9 @@ __global__ void __launch_bounds__(kThreads, 2)
   constexpr int kNewer = (S::kNX - 2) * MF + (S::kNW - 2) * kWi;
   auto wrap = [](uint32_t at, uint32_t by, uint32_t end) { return at + by == end ? 0u : at + by; };
 
-  // F32 results keep short chains of fp32 additions: every kFlush steps the
-  // accumulators are added to a second set and cleared (32 MFMAs of 32 products
-  // to a chain, where the fused GEMM's k quarters have k / 128). bf16 results
-  // are rounded to 8 bits and keep the registers for a wider tile.
-  constexpr uint32_t kFlush = 16;
+  // F32 results keep short chains of fp32 additions: every `flush_steps` steps
+  // the accumulators are added to a second set and cleared. bf16 results are one
+  // chain over the k range and keep the registers for a wider tile.
   f32x4_t sum[F32_OUT ? NF : 1][F32_OUT ? MF : 1];
   auto flush = [&]() {
 #pragma unroll
@@ -207,7 +206,7 @@ __global__ void __launch_bounds__(kThreads, 2)
   }
   publish(std::integral_constant<int, MF + kWi + kNewer>());
   read(f0, 0, 0, 0);
-  uint32_t xat = 0, wat = 0;
+  uint32_t xat = 0, wat = 0, left = flush_steps;
 #pragma unroll 1
   for (uint32_t s = 0; s + 1 < steps; ++s) {
     const uint32_t xn = wrap(xat, S::kX, S::kNX * S::kX), wn_ = wrap(wat, S::kW, S::kNW * S::kW);
@@ -226,7 +225,10 @@ __global__ void __launch_bounds__(kThreads, 2)
     multiply(f1);
     interleave<MF * NF, MF + NF, MF + kWi>();
     if constexpr (F32_OUT) {
-      if ((s + 1) % kFlush == 0) flush();
+      if (--left == 0) {
+        flush();
+        left = flush_steps;
+      }
     }
   }
   read(f1, xat, wat, 1);
@@ -305,6 +307,20 @@ int64_t chunk_rows(int64_t n_rows, int64_t k) {
   return ceil_div(ceil_div(n_rows, ceil_div(n_rows, cap)), 256) * 256;
 }
 
+// Steps between flushes of an F32 product: chains of at most k / 128 MFMAs, the
+// length of the fused GEMM's four k quarters, and of at most 32. Root mean square
+// error against float64, this form over the fused one, Q4_0, 2048 x 2048 outputs,
+// at k = 256, 512, 1024, 2048, 4096 and 14336: 1.00, 1.00, 1.00, 1.00, 1.00 and
+// 0.53 (flushed every 16 steps whatever k: 1.42, 1.68, 1.93, 1.41, 1.00, 0.53; one
+// chain: 1.42, 1.68, 1.93, 2.09, 2.16, 2.15). Four flushes cost up to 1 % of the
+// product's time at k = 1024, eight 2.5 %. The chain of a bf16 result is lost in
+// its rounding: error 1.655e-3 of the outputs in both forms at k = 14336, equal to
+// 1e-7 of itself, and outputs that are not the nearest bf16 5.0e-4 of all against
+// 4.0e-4.
+uint32_t flush_steps(int64_t k) {
+  return static_cast<uint32_t>(std::max<int64_t>(1, std::min<int64_t>(16, k / (4 * kBK))));
+}
+
 template <int MF, int NF, bool F32_OUT>
 int launch(const uint16_t* x, int64_t ldx, int64_t m, const uint16_t* wb, int64_t n, int64_t k, void* y, int64_t ldy,
            hipStream_t s) {
@@ -315,7 +331,8 @@ int launch(const uint16_t* x, int64_t ldx, int64_t m, const uint16_t* wb, int64_
   const int64_t tm = ceil_div(m, 64 * MF), tn = ceil_div(n, 32 * NF);
   hipLaunchKernelGGL((dense_kernel<MF, NF, F32_OUT>), dim3(static_cast<unsigned>(tm * tn)), dim3(kThreads), lds, s, x,
                      static_cast<uint32_t>(ldx), static_cast<uint32_t>(m), wb, static_cast<uint32_t>(n),
-                     static_cast<uint32_t>(k), y, ldy, static_cast<uint32_t>(tm), static_cast<uint32_t>(tn));
+                     static_cast<uint32_t>(k), y, ldy, static_cast<uint32_t>(tm), static_cast<uint32_t>(tn),
+                     flush_steps(k));
   return launch_status();
 }
 
@@ -349,6 +366,9 @@ bool dense_fits(int type, int64_t n_rows, int64_t k, int64_t m, int64_t ldx, boo
   if (m < 256 || n_rows < 256 || k % kBK != 0 || k > (int64_t(1) << 20) || m > (int64_t(1) << 24) ||
       n_rows > (int64_t(1) << 24) || ldx >= (int64_t(1) << 22))
     return false;
+  // Shorter F32 rows: one chain of two or four MFMAs is less exact than the fused
+  // form's quarters (error 1.12 and 1.03 times at k = 64 and 128).
+  if (f32 && k < 192) return false;
   const int64_t wbytes = spiral_tensor_bytes(type, n_rows, k);
   if (wbytes == 0 || wbytes >= (int64_t(1) << 32)) return false;  // the fused GEMM's limit
   const int64_t rounds = ceil_div(ceil_div(m, 128) * ceil_div(n_rows, 64), device_cu_count());

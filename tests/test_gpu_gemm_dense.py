@@ -79,3 +79,39 @@ def test_dense_chunks(cuda):
     sub = np.ascontiguousarray(raw.reshape(n, -1)[rows]).reshape(-1)
     ref = O.matmul_f64(O.dequant(qtype, sub, len(rows), k), x)
     assert rel_err(y[:, rows], ref) <= REL_TOL_EXACT_W
+
+
+# F32 results sum in chains no longer than the fused form's quarters of k, so that
+# rows of a few k steps are as exact. The errors are root mean squares over a
+# million outputs or more, within 1 % of their expectation; one chain every 1024 k
+# had 1.3 to 1.9 times the fused form's at k = 512 to 2048.
+@pytest.mark.parametrize("m,n,k", [(513, 7001, 512), (513, 7001, 1024), (1025, 4097, 512), (1025, 4097, 1024),
+                                   (2049, 4097, 512), (2049, 4097, 1536), (2049, 4097, 2048), (2049, 4097, 4096),
+                                   (2049, 7001, 64), (2049, 7001, 128), (2049, 7001, 192), (2049, 7001, 256)])
+def test_f32_error_at_most_the_fused_forms(cuda, m, n, k):
+    qtype = O.Q4_0
+    w = ops.to_planar(qtype, dev_u8(synth.make_weights(qtype, n, k, 230), cuda), n, k)
+    x = dev_bf16(synth.make_x(m, k, 231), cuda)
+    ref = x.double() @ ops.dequant(qtype, w, n, k).double().t()
+    fused = ops.mul_mat(qtype, w, n, k, x, out_dtype=torch.float32,
+                        workspace=torch.empty(-(-m // 16) * 16 * k * 2, dtype=torch.uint8, device=cuda))
+    y = ops.mul_mat(qtype, w, n, k, x, out_dtype=torch.float32)
+    assert torch.equal(y, fused) == (k < 192)  # shorter rows keep the fused form
+    rms = [float((a.double() - ref).square().mean().sqrt()) for a in (y, fused)]
+    assert rms[0] <= 1.02 * rms[1], rms
+
+
+# A bf16 result is one fp32 chain over k, up to 7e-7 of the outputs from the exact
+# sum; its rounding is 1.66e-3 from it, so the chain adds (7e-7 / 1.66e-3)^2 / 2 =
+# 1e-7 of the error at most.
+@pytest.mark.parametrize("m,n,k", [(513, 7001, 1024), (1025, 7001, 4096), (2049, 7001, 14336)])
+def test_bf16_error_is_the_roundings(cuda, m, n, k):
+    qtype = O.Q4_K
+    w = ops.to_planar(qtype, dev_u8(synth.make_weights(qtype, n, k, 240), cuda), n, k)
+    x = dev_bf16(synth.make_x(m, k, 241), cuda)
+    ref = x.double() @ ops.dequant(qtype, w, n, k).double().t()
+    fused = ops.mul_mat(qtype, w, n, k, x, workspace=torch.empty(-(-m // 16) * 16 * k * 2, dtype=torch.uint8, device=cuda))
+    y = ops.mul_mat(qtype, w, n, k, x)
+    assert not torch.equal(y, fused)
+    rms = [float((a.double() - ref).square().mean().sqrt()) for a in (y, fused)]
+    assert rms[0] <= (1 + 1e-6) * rms[1], rms
