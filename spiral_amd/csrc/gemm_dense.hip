@@ -273,12 +273,12 @@ __global__ void __launch_bounds__(kThreads, 2)
   }
 }
 
-// Tiles (64 MF rows of X x 32 NF rows of W); F32 results need registers for two
-// accumulator sets, so their tiles stop at NF = 5.
+// Tiles (64 MF rows of X x 32 NF rows of W) and their average k step, ns; F32
+// results need registers for two accumulator sets, so their tiles stop at NF = 5.
 struct Tile {
-  int mf, nf;
+  int mf, nf, step_ns;
 };
-constexpr Tile kTiles[] = {{4, 8}, {4, 7}, {4, 6}, {4, 5}, {4, 4}, {2, 4}};
+constexpr Tile kTiles[] = {{4, 8, 1330}, {4, 7, 1200}, {4, 6, 1030}, {4, 5, 960}, {4, 4, 730}, {2, 4, 510}};
 
 // Estimated nanoseconds of the product with tile t: rounds of one workgroup a
 // CU, whose steps take their MFMAs (16 clocks each, two waves a SIMD, and the
@@ -355,15 +355,51 @@ int launch_f32(Tile t, const uint16_t* x, int64_t ldx, int64_t m, const uint16_t
                    : launch<4, 4, true>(x, ldx, m, wb, n, k, y, ldy, s);
 }
 
+// Estimated nanoseconds of the fused GEMM (gemm.hip, one range of k): packing x,
+// then rounds of one 128 x 64 tile a CU, whose time a k follows the format's
+// dequantization; weights that the 256 MiB cache does not hold come from HBM again
+// for every 128 rows.
+int64_t fused_ns(int type, int64_t m, int64_t n, int64_t k, int64_t w_bytes, int64_t y_bytes) {
+  const int64_t tm = ceil_div(m, 128), tiles = tm * ceil_div(n, 64), rounds = ceil_div(tiles, device_cu_count());
+  const int64_t ps = type == SPIRAL_TYPE_Q4_0     ? 3590
+                     : type == SPIRAL_TYPE_Q8_0   ? 3870
+                     : type == SPIRAL_TYPE_IQ4_NL ? 4050
+                     : type == SPIRAL_TYPE_IQ4_XS ? 4240
+                     : type == SPIRAL_TYPE_Q4_K   ? 4400
+                     : type == SPIRAL_TYPE_Q5_K   ? 4710
+                                                  : 4790;
+  return 3560 + 3310 * rounds + 2 * m * k / 4000 + y_bytes / 8450 + tiles * k / 270 + rounds * k * ps / 1000 +
+         tm * std::max<int64_t>(0, w_bytes - 200000000) / 9000;
+}
+
+// Of this form: for each chunk of rows that gemm_dense() takes, its bytes
+// written and read, and the product's rounds at the tile's measured step.
+int64_t dense_ns(int64_t m, int64_t n, int64_t k, bool f32) {
+  const int64_t chunk = chunk_rows(n, k);
+  int64_t ns = 0;
+  for (int64_t r = 0; r < n; r += chunk) {
+    const int64_t nc = std::min(chunk, n - r);
+    const Tile t = choose_tile(m, nc, k, f32);
+    const int64_t rounds = ceil_div(ceil_div(m, 64 * t.mf) * ceil_div(nc, 32 * t.nf), device_cu_count());
+    ns += 7000 + 2 * nc * k / 3500 + m * nc * (f32 ? 4 : 2) / 3200 + rounds * (k / kBK) * t.step_ns;
+  }
+  return ns;
+}
+
 }  // namespace
 
 // Whether the dequantize-once form takes this product: 32-bit row offsets, and
-// estimated to beat the fused GEMM, which takes rounds of one 128 x 64 tile a CU
-// at 5.4 ns a k (Q4_K, k = 4096, us, fused against this form: 4096 x 1024 rows
-// 57 and 49, 14336 x 384 rows 79 and 88, 14336 x 512 100 and 92, 14336 x 2048
-// 348 and 217; k = 14336: 4096 x 1024 164 and 172, 4096 x 2048 326 and 233).
+// estimated to beat the fused GEMM by 4 %. Both estimates were fitted to 2660
+// measured pairs (seven formats, 17 matrices from 1024 x 1024 to 12288 x 36864,
+// 256 to 3072 rows, bf16 and F32); of those and 970 others it sends 44 to a form
+// more than 3 % slower than the fused one (the worst by 12 %). Where they cross,
+// us, fused and this form: Q4_0 4096 x 4096, 768 rows 46 and 51, 1536 rows 73 and
+// 65; Q6_K the same 768 rows 54 and 51; Q4_K 6912 x 2560, 512 rows 37 and 45, 1024
+// rows 70 and 54; Q4_K 16384 x 53248 (eight chunks), 1024 rows 2439 and 4057; Q4_K
+// 49152 x 12288 (five), 512 rows 843 and 1103, 2048 rows 3266 and 2467. No matrix
+// gained at 256 rows: two rows of fused tiles, one of these.
 bool dense_fits(int type, int64_t n_rows, int64_t k, int64_t m, int64_t ldx, bool f32) {
-  if (m < 256 || n_rows < 256 || k % kBK != 0 || k > (int64_t(1) << 20) || m > (int64_t(1) << 24) ||
+  if (m <= 256 || n_rows < 256 || k % kBK != 0 || k > (int64_t(1) << 20) || m > (int64_t(1) << 24) ||
       n_rows > (int64_t(1) << 24) || ldx >= (int64_t(1) << 22))
     return false;
   // Shorter F32 rows: one chain of two or four MFMAs is less exact than the fused
@@ -371,10 +407,7 @@ bool dense_fits(int type, int64_t n_rows, int64_t k, int64_t m, int64_t ldx, boo
   if (f32 && k < 192) return false;
   const int64_t wbytes = spiral_tensor_bytes(type, n_rows, k);
   if (wbytes == 0 || wbytes >= (int64_t(1) << 32)) return false;  // the fused GEMM's limit
-  const int64_t rounds = ceil_div(ceil_div(m, 128) * ceil_div(n_rows, 64), device_cu_count());
-  const int64_t fused = rounds * (k * 54 / 10 + 2000) + 6000;
-  const int64_t dense = (wbytes + 2 * n_rows * k) / 5200 + 2000 + tile_ns(choose_tile(m, n_rows, k, f32), m, n_rows, k);
-  return dense < fused;
+  return dense_ns(m, n_rows, k, f32) * 104 < fused_ns(type, m, n_rows, k, wbytes, m * n_rows * (f32 ? 4 : 2)) * 100;
 }
 
 int64_t dense_workspace_bytes(int64_t n_rows, int64_t k) { return chunk_rows(n_rows, k) * k * 2; }

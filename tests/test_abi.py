@@ -232,3 +232,29 @@ def test_glu_fits_predicate(spiral_lib):
     assert L.spiral_mul_mat_id_glu_fits(q6, 64, 2048) == 1
     assert L.spiral_mul_mat_id_glu_fits(q6, 64, 2048 + 32) == 0
     assert L.spiral_mul_mat_id_glu_fits(_lib.TYPE_F32, 64, 2048) == 0
+
+
+# Which form a product of many rows takes follows from its workspace: the packed x
+# (fused GEMM) or the dequantized rows of a chunk (dequantized once). us, fused and
+# dequantized once, as measured; the first six were sent to the slower form while
+# one estimate stood for all formats and for a matrix taken in chunks.
+@pytest.mark.parametrize("qtype,m,n,k,dense", [
+    (O.Q4_K, 640, 16384, 53248, False),   # eight chunks: 1773 and 4131
+    (O.Q4_K, 512, 49152, 12288, False),   # five: 843 and 1103
+    (O.Q4_K, 768, 12288, 36864, False),   # four: 1004 and 1536
+    (O.Q4_0, 768, 4096, 4096, False),     # 46 and 51
+    (O.IQ4_XS, 384, 6912, 2560, False),   # 35 and 45
+    (O.Q4_K, 256, 32768, 512, False),     # 31 and 38
+    (O.Q6_K, 768, 4096, 4096, True),      # 54 and 51
+    (O.Q4_0, 1536, 4096, 4096, True),     # 73 and 65
+    (O.Q4_K, 1024, 65536, 4096, True),    # 824 and 533, two chunks
+    (O.Q4_K, 2048, 49152, 12288, True),   # 3266 and 2467, five
+    (O.Q4_K, 2048, 14336, 4096, True),    # 369 and 205
+])
+def test_many_row_form_is_the_faster_one(spiral_lib, qtype, m, n, k, dense):
+    need = spiral_lib.spiral_mul_mat_workspace_bytes(qtype, n, k, m)
+    packed = -(-m // 16) * 16 * k * 2
+    if not dense:
+        assert need == packed
+    else:
+        assert need > packed and need % (2 * k) == 0 and need <= 256 << 20
