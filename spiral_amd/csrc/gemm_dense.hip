@@ -300,7 +300,8 @@ Tile choose_tile(int64_t m, int64_t n, int64_t k, bool f32) {
 
 constexpr int64_t kMaxChunkBytes = int64_t(256) << 20;
 
-// Weight rows dequantized at a time: all of them up to 256 MiB of bf16.
+// Weight rows dequantized at a time: all of them up to 256 MiB of bf16 (256 rows
+// at least, which dense_fits() holds below that).
 int64_t chunk_rows(int64_t n_rows, int64_t k) {
   const int64_t cap = std::max<int64_t>(kMaxChunkBytes / (2 * k) / 256 * 256, 256);
   if (n_rows <= cap) return n_rows;
@@ -399,7 +400,7 @@ int64_t dense_ns(int64_t m, int64_t n, int64_t k, bool f32) {
 // 49152 x 12288 (five), 512 rows 843 and 1103, 2048 rows 3266 and 2467. No matrix
 // gained at 256 rows: two rows of fused tiles, one of these.
 bool dense_fits(int type, int64_t n_rows, int64_t k, int64_t m, int64_t ldx, bool f32) {
-  if (m <= 256 || n_rows < 256 || k % kBK != 0 || k > (int64_t(1) << 20) || m > (int64_t(1) << 24) ||
+  if (m <= 256 || n_rows < 256 || k % kBK != 0 || k > kMaxChunkBytes / 512 || m > (int64_t(1) << 24) ||
       n_rows > (int64_t(1) << 24) || ldx >= (int64_t(1) << 22))
     return false;
   // Shorter F32 rows: one chain of two or four MFMAs is less exact than the fused
