@@ -168,7 +168,10 @@ __device__ __forceinline__ void gemm_step(f32x4_t (&acc)[4][4], Pipe<TYPE>& pp, 
   __builtin_amdgcn_sched_barrier(0);
 }
 
-template <int TYPE, bool F32_OUT>
+// SPLIT: ranges of k (below). A kernel of its own: with the range's arithmetic in
+// every product, the unsplit ones took 0.4 to 1.8 % more time at k >= 2048 and 2 to
+// 3.7 % at k = 256.
+template <int TYPE, bool F32_OUT, bool SPLIT>
 __global__ void __launch_bounds__(kThreads) gemm_kernel(const uint8_t* __restrict__ w, int64_t n_rows, int64_t k,
                                                         const uint16_t* __restrict__ xp, int64_t m,
                                                         void* __restrict__ y, int64_t ldy, int64_t n_tiles_n,
@@ -185,15 +188,22 @@ __global__ void __launch_bounds__(kThreads) gemm_kernel(const uint8_t* __restric
   const int64_t nb = k / block_elems(TYPE);
   // 32-bit step counters keep the ring's clamps scalar (k is at most
   // gemm_max_k(), so k / 128 fits)
-  // Workgroup (b, z) of Z = gridDim.y takes the z-th of Z ranges of k steps
-  // (whole pairs of steps: super-blocks), `full` steps from step kb, and writes
-  // to y + z * y_split; the last range has the k tail. The range's start goes
-  // into the lanes' offsets, so the loop counts from 0.
-  const int all = static_cast<int>(k / kBK), z = blockIdx.y, nz = gridDim.y;
-  const int kb = static_cast<int>(static_cast<int64_t>(all / 2) * z / nz) * 2;
-  const bool last = z + 1 == nz;
-  const int full = (last ? all : static_cast<int>(static_cast<int64_t>(all / 2) * (z + 1) / nz) * 2) - kb;
-  const int tail = last ? static_cast<int>(k - static_cast<int64_t>(all) * kBK) : 0;  // 0, 32, 64 or 96
+  int kb = 0, full = static_cast<int>(k / kBK), z = 0;
+  int tail = static_cast<int>(k - static_cast<int64_t>(full) * kBK);  // 0, 32, 64 or 96
+  if constexpr (SPLIT) {
+    // Workgroup (b, z) of Z = gridDim.y takes the z-th of Z ranges of k steps
+    // (whole pairs of steps: super-blocks), `full` steps from step kb, and writes
+    // to y + z * y_split; the last range has the k tail. The range's start goes
+    // into the lanes' offsets, so the loop counts from 0.
+    const int pairs = full / 2, nz = gridDim.y;
+    z = blockIdx.y;
+    kb = static_cast<int>(static_cast<int64_t>(pairs) * z / nz) * 2;
+    if (z + 1 < nz) {
+      full = static_cast<int>(static_cast<int64_t>(pairs) * (z + 1) / nz) * 2;
+      tail = 0;
+    }
+    full -= kb;
+  }
   const int64_t kk_n = k >> 5, mb_n = (m + 15) >> 4;
   const __amdgpu_buffer_rsrc_t X = buffer_rsrc(xp, static_cast<uint32_t>(mb_n * kk_n * 1024));
   uint32_t voff[4];
@@ -202,7 +212,7 @@ __global__ void __launch_bounds__(kThreads) gemm_kernel(const uint8_t* __restric
     voff[i] = static_cast<uint32_t>((min((row0 >> 4) + i, mb_n - 1) * kk_n + 4 * kb) * 1024 + lane * 16);
   const Planes P = make_planes<TYPE>(w, n_rows, nb);
   typename Piece<TYPE>::Addr pa = Piece<TYPE>::addr(min(n0 + (tid >> 3), n_rows - 1), nb, tid & 7);
-  Piece<TYPE>::skip(pa, static_cast<uint32_t>(kb));
+  if constexpr (SPLIT) Piece<TYPE>::skip(pa, static_cast<uint32_t>(kb));
 
   f32x4_t acc[4][4];
 #pragma unroll
@@ -390,19 +400,23 @@ int launch_gemm(const void* w, int64_t n_rows, int64_t k, const uint16_t* x, int
     const int64_t nz = k_splits(m, n_rows, k);
     if (nz > 1 && workspace_bytes >= gemm_workspace_bytes(m, n_rows, k)) {  // one chunk
       float* part = reinterpret_cast<float*>(reinterpret_cast<uint8_t*>(xp) + packed_bytes(m, k));
-      hipLaunchKernelGGL((gemm_kernel<TYPE, true>), dim3(grid.x, static_cast<unsigned>(nz)), dim3(kThreads), 0, s, W,
-                         n_rows, k, xp, m, part, n_rows, tn, m * n_rows);
+      hipLaunchKernelGGL((gemm_kernel<TYPE, true, true>), dim3(grid.x, static_cast<unsigned>(nz)), dim3(kThreads), 0,
+                         s, W, n_rows, k, xp, m, part, n_rows, tn, m * n_rows);
       rc = launch_status();
       if (rc != SPIRAL_OK) return rc;
       const dim3 sums(static_cast<unsigned>(ceil_div(m * n_rows, 1024)));
       if (y_type == SPIRAL_TYPE_F32)
-        hipLaunchKernelGGL(sum_splits_kernel<true>, sums, dim3(256), 0, s, part, static_cast<int>(nz), m, n_rows, y, ldy);
+        hipLaunchKernelGGL(sum_splits_kernel<true>, sums, dim3(256), 0, s, part, static_cast<int>(nz), m, n_rows, y,
+                           ldy);
       else
-        hipLaunchKernelGGL(sum_splits_kernel<false>, sums, dim3(256), 0, s, part, static_cast<int>(nz), m, n_rows, y, ldy);
+        hipLaunchKernelGGL(sum_splits_kernel<false>, sums, dim3(256), 0, s, part, static_cast<int>(nz), m, n_rows, y,
+                           ldy);
     } else if (y_type == SPIRAL_TYPE_F32) {
-      hipLaunchKernelGGL((gemm_kernel<TYPE, true>), grid, dim3(kThreads), 0, s, W, n_rows, k, xp, mc, yc, ldy, tn, 0);
+      hipLaunchKernelGGL((gemm_kernel<TYPE, true, false>), grid, dim3(kThreads), 0, s, W, n_rows, k, xp, mc, yc, ldy,
+                         tn, 0);
     } else {
-      hipLaunchKernelGGL((gemm_kernel<TYPE, false>), grid, dim3(kThreads), 0, s, W, n_rows, k, xp, mc, yc, ldy, tn, 0);
+      hipLaunchKernelGGL((gemm_kernel<TYPE, false, false>), grid, dim3(kThreads), 0, s, W, n_rows, k, xp, mc, yc, ldy,
+                         tn, 0);
     }
     rc = launch_status();
     if (rc != SPIRAL_OK) return rc;
