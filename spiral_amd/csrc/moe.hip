@@ -57,7 +57,8 @@
 #include "moe_piece.h"
 
 namespace spiral {
-bool moe_tile_fits(int type, int64_t n_expert, int64_t k, int64_t x_slots, int64_t n_pairs, int64_t top_k);
+bool moe_tile_fits(int type, int64_t n_expert, int64_t n_rows, int64_t k, int64_t x_slots, int64_t n_pairs,
+                   int64_t top_k, bool short_rows);
 int moe_tile(int type, const void* w, const void* w_up, int64_t expert_stride, int64_t n_expert, int64_t n_rows,
              int64_t k, const uint16_t* x, int64_t x_slots, int64_t n_pairs, int64_t top_k, const int32_t* offsets,
              const int32_t* list, void* y, bool f32, int glu_op, int swapped, hipStream_t s);
@@ -1551,7 +1552,8 @@ int moe(int type, const void* w, int64_t expert_stride, int64_t n_expert, int64_
   if (glu && !stream_ok) return SPIRAL_ERR_SHAPE;
   int32_t* offsets = nullptr;
   int32_t* list = nullptr;
-  const bool tiled = moe_tile_fits(type, n_expert, k, x_slots, n_pairs, top_k);
+  const bool short_rows = !glu && stream_ok && stream_lds_bytes(k, 4) > 0;
+  const bool tiled = moe_tile_fits(type, n_expert, n_rows, k, x_slots, n_pairs, top_k, short_rows);
   if (n_pairs > kFusedPairs || tiled) {
     offsets = static_cast<int32_t*>(workspace);
     list = offsets + n_expert + 1;

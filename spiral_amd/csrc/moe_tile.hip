@@ -379,10 +379,24 @@ int launch_tile(const void* w, const void* w_up, int64_t expert_stride, int64_t 
 // 199 and 173; IQ4_XS 159 and 189, 210 and 185, 267 and 194. Past k = 2304 its
 // passes stay at 16: 60 experts, 3072 / 1536, 13 tokens: Q4_K 310 and 221, Q4_0
 // 246 and 203, IQ4_XS 264 and 239.
-bool moe_tile_fits(int type, int64_t n_expert, int64_t k, int64_t x_slots, int64_t n_pairs, int64_t top_k) {
+//
+// short_rows: a product without GLU whose rows leave LDS for the streaming form's
+// passes of 64 tokens. It stays with that form while the average expert fills at
+// most 0.7 of its passes, so that evenly routed experts take one pass each, side
+// by side (for several passes, while there are row groups enough for the chip):
+// 128 experts of 2048 x 768, us, streaming and this form at 36, 40, 48, 56, 80 and
+// 128 tokens an expert, Q4_K 51 and 70, 52 and 72, 80 and 73, 82 and 78, 95 and 112,
+// 139 and 152; Q4_0 50 and 71, 51 and 73, 74 and 74, 74 and 78, 93 and 117, 130 and
+// 154. An expert of several times the average takes its passes one after another
+// there: with popularities spread over e^0.25 (the busiest of 128 at twice the
+// average) the two forms meet, over e^0.5 this one leads (40 tokens: 92 and 73).
+bool moe_tile_fits(int type, int64_t n_expert, int64_t n_rows, int64_t k, int64_t x_slots, int64_t n_pairs,
+                   int64_t top_k, bool short_rows) {
   if (type != SPIRAL_TYPE_Q4_0 && !is_iq4(type) && !is_kquant(type)) return false;
   if (k % 256 != 0 || n_expert > 65535 || n_pairs / top_k * x_slots * k * 2 >= (int64_t(1) << 31)) return false;
-  return n_pairs >= (k > 2304 ? 13 : 24) * n_expert;
+  if (n_pairs < (k > 2304 ? 13 : 24) * n_expert) return false;
+  const int64_t avg = ceil_div(n_pairs, n_expert), passes = ceil_div(avg, 64);
+  return !(short_rows && avg > 32 && 10 * avg <= 7 * 64 * passes && (passes == 1 || n_expert * n_rows >= 120000));
 }
 
 // Arguments validated by the caller (moe); offsets and list from the route kernel.

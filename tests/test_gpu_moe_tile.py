@@ -92,3 +92,30 @@ def test_tile_slots_and_many_tiles(cuda, qtype):
     y = call(xd, idd)
     assert torch.equal(y, small_calls(call, xd, idd, 10))
     check_moe(y.cpu().numpy(), _moe_ref(qtype, raws, n, k, ids, x), True)
+
+
+# Which form ran shows in the workspace: with at most 1024 pairs only the tiled
+# form has the routing lists written there. Rows of up to 1152 k stay with the
+# streaming form while its passes of 64 tokens hold the average expert with room
+# (33 to 44 tokens; 65 to 89 with many rows), which is the faster one there.
+@pytest.mark.parametrize("e,n,k,per,tiled", [
+    (8, 96, 768, 23, False), (8, 96, 768, 24, True), (8, 96, 768, 32, True), (8, 96, 768, 33, False),
+    (8, 96, 1024, 44, False), (8, 96, 768, 45, True), (8, 96, 768, 64, True), (8, 96, 768, 72, True),
+    (8, 15000, 768, 64, True), (8, 15000, 768, 65, False), (8, 15000, 512, 89, False), (8, 15000, 512, 90, True),
+    (8, 96, 1280, 40, True), (8, 96, 2560, 13, True), (8, 96, 2560, 12, False),
+])
+def test_form_by_tokens_an_expert(cuda, e, n, k, per, tiled):
+    qtype, tokens = O.Q4_K, per * e
+    w = torch.zeros((e, O.row_bytes(qtype, k) * n), dtype=torch.uint8, device=cuda)
+    x = torch.ones((tokens, 1, k), dtype=torch.bfloat16, device=cuda)
+    ids = (torch.arange(tokens, dtype=torch.int32, device=cuda) % e)[:, None].contiguous()
+    ws = torch.full((4 * (e + 1 + tokens),), 0x5A, dtype=torch.uint8, device=cuda)
+    y = ops.mul_mat_id(qtype, w, w.stride(0), e, n, k, x, ids, out_dtype=torch.float32, workspace=ws)
+    torch.cuda.synchronize()
+    assert bool((ws != 0x5A).any()) == tiled
+    assert not y.any()
+    if k <= 1152:  # the fused GLU form's passes take 32 tokens at most: tiled from 24 on
+        ws.fill_(0x5A)
+        ops.mul_mat_id_glu(qtype, w, w.stride(0), e, n, k, x, ids, ops.GLU_SWIGLU, workspace=ws)
+        torch.cuda.synchronize()
+        assert bool((ws != 0x5A).any()) == (per >= 24)
