@@ -4,8 +4,9 @@ format it has, rows
 that are no multiple of its 96 (48 features with GLU), of 16 or of 4, one to five
 super-blocks of k, experts of no tokens, of one, and of counts at the edges of
 its token tiles (32, 64, 80 and over), per-slot inputs, ids routed nowhere, the
-fused GLU form merged and split. Equal bit for bit to the same tokens in small
-calls (the streaming form), and to the oracle within the product bars.
+fused GLU form merged and split, every GLU variant. Up to k = 4096 equal bit for
+bit to the same tokens in small calls (the streaming form, which ends there), and
+to the oracle within the product bars at every k.
 """
 
 import numpy as np
@@ -119,3 +120,52 @@ def test_form_by_tokens_an_expert(cuda, e, n, k, per, tiled):
         ops.mul_mat_id_glu(qtype, w, w.stride(0), e, n, k, x, ids, ops.GLU_SWIGLU, workspace=ws)
         torch.cuda.synchronize()
         assert bool((ws != 0x5A).any()) == (per >= 24)
+
+
+@pytest.mark.parametrize("per", [13, 16, 23])
+@pytest.mark.parametrize("k", [2560, 4096, 5120])
+@pytest.mark.parametrize("qtype", FORMATS)
+def test_tile_long_rows(cuda, qtype, k, per):
+    """13 to 23 tokens an expert, tiled past k = 2304; past 4096 the small calls
+    run another kernel, whose sums are ordered otherwise."""
+    e, n, tokens = 3, 100, 3 * per
+    ids = (np.arange(tokens, dtype=np.int32) % e)[:, None]
+    w, per_e, raws, ids, x = _moe_inputs(cuda, qtype, e, n, k, tokens, 1, 1, 430, ids)
+    xd, idd = dev_bf16(x, cuda), torch.from_numpy(ids).to(cuda)
+    ws = torch.zeros(4 * (e + 1 + tokens), dtype=torch.uint8, device=cuda)
+
+    def call(xs, i, ws=None):
+        return ops.mul_mat_id(qtype, w, per_e, e, n, k, xs, i, out_dtype=torch.float32, workspace=ws)
+
+    y = call(xd, idd, ws)
+    assert ws.any()  # the tiled form's routing lists
+    if k <= 4096:
+        assert torch.equal(y, small_calls(call, xd, idd, 10))
+    check_moe(y.cpu().numpy(), _moe_ref(qtype, raws, n, k, ids, x), True)
+
+
+@pytest.mark.parametrize("split", [False, True])
+@pytest.mark.parametrize("swapped", [False, True])
+@pytest.mark.parametrize("op", [ops.GLU_REGLU, ops.GLU_GEGLU, ops.GLU_SWIGLU, ops.GLU_GEGLU_ERF, ops.GLU_GEGLU_QUICK])
+def test_tile_glu_variants(cuda, op, swapped, split):
+    """Every activation, merged and split, halves swapped: the product and the
+    standalone GLU bit for bit; bf16 output its rounding."""
+    qtype, e, F, k, tokens, top = O.Q4_K, 4, 56, 512, 120, 2
+    n = 2 * F
+    w, per, raws, ids, x = _moe_inputs(cuda, qtype, e, n, k, tokens, top, 1, 440)
+    xd, idd = dev_bf16(x, cuda), torch.from_numpy(ids).to(cuda)
+    prod = ops.mul_mat_id(qtype, w, per, e, n, k, xd, idd, out_dtype=torch.float32)
+    if split:
+        half = [torch.stack([ops.to_planar(qtype, torch.from_numpy(np.ascontiguousarray(
+            r.reshape(n, -1)[i * F:(i + 1) * F]).reshape(-1)).to(cuda), F, k) for r in raws]) for i in range(2)]
+        want = ops.glu_split(prod[..., :F].contiguous(), prod[..., F:].contiguous(), op, swapped)
+    else:
+        want = ops.glu(prod, op, swapped)
+    for dtype in (torch.float32, torch.bfloat16):
+        if split:
+            got = ops.mul_mat_id_glu_split(qtype, half[0], half[1], half[0].shape[1], e, F, k, xd, idd, op, swapped,
+                                           out_dtype=dtype)
+        else:
+            got = ops.mul_mat_id_glu(qtype, w, per, e, n, k, xd, idd, op, swapped, out_dtype=dtype)
+        torch.cuda.synchronize()
+        assert torch.equal(got, want.to(dtype))
