@@ -35,6 +35,17 @@ bool glu_op_ok(int op) {
          op == SPIRAL_GLU_GEGLU_ERF || op == SPIRAL_GLU_GEGLU_QUICK;
 }
 
+// Products that need no workspace: the GEMV and the small-batch form.
+bool runs_direct(int type, int64_t n_rows, int64_t k, int64_t m) {
+  return (m == 1 && k <= gemv_max_k(type, true)) || skinny_fits(type, n_rows, k, m);
+}
+
+// The least workspace a call takes is the fused GEMM's; the forms that want more
+// run when the caller's workspace holds it.
+int64_t mul_mat_least_workspace(int type, int64_t n_rows, int64_t k, int64_t m) {
+  return runs_direct(type, n_rows, k, m) ? 0 : gemm_min_workspace_bytes(m, k);
+}
+
 // Checks shared by MUL_MAT_ID and its fused GLU form.
 int check_mul_mat_id(int type, const void* w, int64_t expert_stride, int64_t n_expert, int64_t n_rows, int64_t k,
                      const uint16_t* x, int64_t x_slots, const int32_t* ids, int64_t n_tokens, int64_t top_k,
@@ -65,8 +76,7 @@ extern "C" {
 
 int64_t spiral_mul_mat_workspace_bytes(int type, int64_t n_rows, int64_t k, int64_t m) {
   if (!is_quant_type(type) || n_rows <= 0 || m <= 0 || k <= 0 || k % block_elems(type) != 0) return 0;
-  if (m == 1 && k <= gemv_max_k(type, true)) return 0;
-  if (skinny_fits(type, n_rows, k, m)) return 0;
+  if (runs_direct(type, n_rows, k, m)) return 0;
   const int64_t need = gemm_workspace_bytes(m, n_rows, k);  // 0 past the GEMM's longest row: spiral_mul_mat refuses that shape
   const bool dense = need > 0 && (dense_fits(type, n_rows, k, m, k, false) || dense_fits(type, n_rows, k, m, k, true));
   return dense ? std::max(need, dense_workspace_bytes(n_rows, k)) : need;
@@ -82,11 +92,9 @@ int spiral_mul_mat(int type, const void* w, int64_t n_rows, int64_t k, const uin
   if (ldx < k || ldy < n_rows || spiral_tensor_bytes(type, n_rows, k) == 0) return SPIRAL_ERR_SHAPE;
   if (!aligned16(w) || !aligned16(x) || ldx % 8 != 0) return SPIRAL_ERR_ALIGN;
   if ((reinterpret_cast<uintptr_t>(y) & 3u) != 0) return SPIRAL_ERR_ALIGN;
-  const bool direct = (m == 1 && k <= gemv_max_k(type, true)) || skinny_fits(type, n_rows, k, m);
+  const bool direct = runs_direct(type, n_rows, k, m);
   if (!direct && k > gemm_max_k()) return SPIRAL_ERR_SHAPE;
-  // The least workspace a call takes is the fused GEMM's; the forms that want
-  // more run when the caller's workspace holds it.
-  const int64_t need = direct ? 0 : gemm_min_workspace_bytes(m, k);
+  const int64_t need = mul_mat_least_workspace(type, n_rows, k, m);
   if (need > 0) {
     if (workspace == nullptr) return SPIRAL_ERR_NULL;
     if (workspace_bytes < need) return SPIRAL_ERR_CAPACITY;

@@ -13,6 +13,7 @@
 #include <new>
 
 #include "common.h"
+#include "scratch.h"
 #include "spiral_ggml.h"
 
 struct spiral_buffer {
@@ -24,8 +25,7 @@ struct spiral_buffer {
 struct spiral_backend {
   int device;
   hipStream_t stream;
-  uint8_t* scratch;
-  size_t scratch_size;
+  spiral::Scratch scratch;
 };
 
 namespace spiral {
@@ -204,16 +204,18 @@ size_t act_scratch(const spiral_tensor* b) {
 }
 
 // Workspace of one MUL_MAT product (the batch's matrices run one after
-// another on the backend's stream and share it).
-size_t mul_mat_workspace(const spiral_tensor* t) {
+// another on the backend's stream and share it); least: what it cannot do without.
+size_t mul_mat_workspace(const spiral_tensor* t, bool least) {
   const spiral_tensor* a = t->src[0];
-  const int64_t n = spiral_mul_mat_workspace_bytes(a->type, a->ne[1], a->ne[0], t->src[1]->ne[1]);
+  const int64_t m = t->src[1]->ne[1];
+  const int64_t n = least ? mul_mat_least_workspace(a->type, a->ne[1], a->ne[0], m)
+                          : spiral_mul_mat_workspace_bytes(a->type, a->ne[1], a->ne[0], m);
   return align_up(static_cast<size_t>(n > 0 ? n : 0), kAlign);
 }
 
-size_t node_scratch(const spiral_tensor* t) {
+size_t node_scratch(const spiral_tensor* t, bool least) {
   switch (t->op) {
-    case SPIRAL_OP_MUL_MAT: return act_scratch(t->src[1]) + mul_mat_workspace(t);
+    case SPIRAL_OP_MUL_MAT: return act_scratch(t->src[1]) + mul_mat_workspace(t, least);
     case SPIRAL_OP_MUL_MAT_ID: {
       const spiral_tensor* b = t->src[1];
       const spiral_tensor* ids = t->src[2];
@@ -269,13 +271,13 @@ int compute_mul_mat(spiral_backend* be, const spiral_tensor* t, const spiral_ten
   const spiral_tensor* b = t->src[1];
   int rc = SPIRAL_OK;
   int64_t ld1 = b->ne[0], ld2 = ld1 * b->ne[1], ld3 = ld2 * b->ne[2];
-  const uint16_t* xb = reinterpret_cast<const uint16_t*>(be->scratch);
+  const uint16_t* xb = reinterpret_cast<const uint16_t*>(be->scratch.base);
   // The workspace lies behind the activation's copy. Rows read in place have
   // none, so there it is the start of the scratch, where a held copy lies.
-  uint8_t* ws = be->scratch + act_scratch(b);
-  const int64_t wsb = static_cast<int64_t>(mul_mat_workspace(t));
+  uint8_t* ws = be->scratch.base + act_scratch(b);
+  const int64_t wsb = static_cast<int64_t>(std::min(mul_mat_workspace(t, false), be->scratch.size - act_scratch(b)));
   if (held != b) {
-    xb = act_bf16(b, be->scratch, false, be->stream, ld1, ld2, ld3, rc);
+    xb = act_bf16(b, be->scratch.base, false, be->stream, ld1, ld2, ld3, rc);
     if (rc != SPIRAL_OK) return rc;
     if (act_scratch(b) != 0)
       held = b;
@@ -322,13 +324,13 @@ int compute_mul_mat_id(spiral_backend* be, const spiral_tensor* t) {
   const spiral_tensor* ids = t->src[2];
   int rc;
   int64_t ld1, ld2, ld3;
-  const uint16_t* x = act_bf16(b, be->scratch, true, be->stream, ld1, ld2, ld3, rc);
+  const uint16_t* x = act_bf16(b, be->scratch.base, true, be->stream, ld1, ld2, ld3, rc);
   if (rc != SPIRAL_OK) return rc;
   const size_t xbytes = align_up(static_cast<size_t>(b->ne[0] * b->ne[1] * b->ne[2]) * 2, kAlign);
   const int64_t wsb = spiral_mul_mat_id_workspace_bytes(a->ne[2], ids->ne[1], ids->ne[0]);
   return spiral_mul_mat_id(a->type, a->data, static_cast<int64_t>(a->nb[2]), a->ne[2], a->ne[1], a->ne[0], x,
                            b->ne[1], static_cast<const int32_t*>(ids->data), ids->ne[1], ids->ne[0], t->data,
-                           SPIRAL_TYPE_F32, be->scratch + xbytes, wsb, be->stream);
+                           SPIRAL_TYPE_F32, be->scratch.base + xbytes, wsb, be->stream);
 }
 
 // MUL_MAT_ID node t with the GLU node g over it as one pass: g's data
@@ -339,13 +341,14 @@ int compute_mul_mat_id_glu(spiral_backend* be, const spiral_tensor* t, const spi
   const spiral_tensor* ids = t->src[2];
   int rc;
   int64_t ld1, ld2, ld3;
-  const uint16_t* x = act_bf16(b, be->scratch, true, be->stream, ld1, ld2, ld3, rc);
+  const uint16_t* x = act_bf16(b, be->scratch.base, true, be->stream, ld1, ld2, ld3, rc);
   if (rc != SPIRAL_OK) return rc;
   const size_t xbytes = align_up(static_cast<size_t>(b->ne[0] * b->ne[1] * b->ne[2]) * 2, kAlign);
   const int64_t wsb = spiral_mul_mat_id_workspace_bytes(a->ne[2], ids->ne[1], ids->ne[0]);
   return spiral_mul_mat_id_glu(a->type, a->data, static_cast<int64_t>(a->nb[2]), a->ne[2], a->ne[1], a->ne[0], x,
                                b->ne[1], static_cast<const int32_t*>(ids->data), ids->ne[1], ids->ne[0],
-                               g->op_params[0], g->op_params[1], g->data, SPIRAL_TYPE_F32, be->scratch + xbytes, wsb,
+                               g->op_params[0], g->op_params[1], g->data, SPIRAL_TYPE_F32,
+                               be->scratch.base + xbytes, wsb,
                                be->stream);
 }
 
@@ -385,14 +388,14 @@ int compute_mul_mat_id_glu_split(spiral_backend* be, const spiral_tensor* g) {
   const spiral_tensor* ids = tg->src[2];
   int rc;
   int64_t ld1, ld2, ld3;
-  const uint16_t* x = act_bf16(b, be->scratch, true, be->stream, ld1, ld2, ld3, rc);
+  const uint16_t* x = act_bf16(b, be->scratch.base, true, be->stream, ld1, ld2, ld3, rc);
   if (rc != SPIRAL_OK) return rc;
   const size_t xbytes = align_up(static_cast<size_t>(b->ne[0] * b->ne[1] * b->ne[2]) * 2, kAlign);
   const int64_t wsb = spiral_mul_mat_id_workspace_bytes(a->ne[2], ids->ne[1], ids->ne[0]);
   return spiral_mul_mat_id_glu_split(a->type, a->data, tu->src[0]->data, static_cast<int64_t>(a->nb[2]), a->ne[2],
                                      a->ne[1], a->ne[0], x, b->ne[1], static_cast<const int32_t*>(ids->data),
                                      ids->ne[1], ids->ne[0], g->op_params[0], 0, g->data, SPIRAL_TYPE_F32,
-                                     be->scratch + xbytes, wsb, be->stream);
+                                     be->scratch.base + xbytes, wsb, be->stream);
 }
 
 // Node i (MUL_MAT_ID) can run fused with node i + 1 (GLU over it): nothing
@@ -455,7 +458,7 @@ uint16_t* copy_for_next(const spiral_backend* be, const spiral_cgraph* graph, in
   if (i + 1 >= graph->n_nodes || t->type != SPIRAL_TYPE_F32) return nullptr;
   const spiral_tensor* next = graph->nodes[i + 1];
   if (next->op != SPIRAL_OP_MUL_MAT || next->src[1] != t) return nullptr;
-  return reinterpret_cast<uint16_t*>(be->scratch);
+  return reinterpret_cast<uint16_t*>(be->scratch.base);
 }
 
 // Whether node t's output shares memory with `b` (strided extents).
@@ -469,19 +472,18 @@ bool overlaps(const spiral_tensor* t, const spiral_tensor* b) {
   return p < q + extent(b) && q < p + extent(t);
 }
 
-int grow_scratch(spiral_backend* be, size_t need) {
-  if (need <= be->scratch_size) return SPIRAL_OK;
-  int rc = hip_rc(hipStreamSynchronize(be->stream));
+// Scratch of `need` bytes, or of `least` (what the graph cannot do without) where
+// the device has no room for them: the products then run their forms of less
+// memory (compute_mul_mat).
+int grow_scratch(spiral_backend* be, size_t need, size_t least) {
+  if (need <= be->scratch.size) return SPIRAL_OK;
+  const int rc = hip_rc(hipStreamSynchronize(be->stream));
   if (rc != SPIRAL_OK) return rc;
-  if (be->scratch != nullptr) (void)hipFree(be->scratch);
-  be->scratch = nullptr;
-  be->scratch_size = 0;
-  void* p = nullptr;
-  rc = hip_rc(hipMalloc(&p, need));
-  if (rc != SPIRAL_OK) return rc;
-  be->scratch = static_cast<uint8_t*>(p);
-  be->scratch_size = need;
-  return SPIRAL_OK;
+  const auto alloc = [](size_t n) {
+    void* p = nullptr;
+    return hip_rc(hipMalloc(&p, n)) == SPIRAL_OK ? p : nullptr;
+  };
+  return grow(be->scratch, need, least, alloc, [](void* p) { (void)hipFree(p); }) ? SPIRAL_OK : SPIRAL_ERR_HIP;
 }
 
 // Runs on the device that owns `buf`, restoring the caller's device.
@@ -732,7 +734,7 @@ spiral_backend* spiral_backend_init(int device) {
     (void)hipGetLastError();
     return nullptr;
   }
-  spiral_backend* be = new (std::nothrow) spiral_backend{device, s, nullptr, 0};
+  spiral_backend* be = new (std::nothrow) spiral_backend{device, s, {}};
   if (be == nullptr) (void)hipStreamDestroy(s);
   return be;
 }
@@ -741,7 +743,7 @@ void spiral_backend_free(spiral_backend* be) {
   if (be == nullptr) return;
   DeviceGuard g(be->device);
   (void)hipStreamSynchronize(be->stream);
-  if (be->scratch != nullptr) (void)hipFree(be->scratch);
+  if (be->scratch.base != nullptr) (void)hipFree(be->scratch.base);
   (void)hipStreamDestroy(be->stream);
   delete be;
 }
@@ -753,15 +755,16 @@ void* spiral_backend_stream(const spiral_backend* be) { return be == nullptr ? n
 int spiral_backend_graph_compute(spiral_backend* be, const spiral_cgraph* graph) {
   if (be == nullptr || graph == nullptr) return SPIRAL_ERR_NULL;
   if (graph->n_nodes > 0 && graph->nodes == nullptr) return SPIRAL_ERR_NULL;
-  size_t need = 0;
+  size_t need = 0, least = 0;
   for (int32_t i = 0; i < graph->n_nodes; ++i) {
     const spiral_tensor* t = graph->nodes[i];
     if (t == nullptr) return SPIRAL_ERR_NULL;
     if (!spiral_supports_op(t)) return SPIRAL_ERR_TYPE;
-    need = std::max(need, node_scratch(t));
+    need = std::max(need, node_scratch(t, false));
+    least = std::max(least, node_scratch(t, true));
   }
   DeviceGuard g(be->device);
-  int rc = grow_scratch(be, need);
+  int rc = grow_scratch(be, need, least);
   if (rc != SPIRAL_OK) return rc;
   const spiral_tensor* held = nullptr;  // see compute_mul_mat
   for (int32_t i = 0; i < graph->n_nodes && rc == SPIRAL_OK; ++i) {

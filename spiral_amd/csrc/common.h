@@ -276,6 +276,9 @@ int blocks_per_cu(const void* kernel, int threads, int64_t lds);
 // (hipFuncSetAttribute once per device and kernel, thread-safe).
 int allow_dynamic_lds(const void* kernel, int bytes);
 
+// The least workspace spiral_mul_mat takes (api.hip); with more it may run a faster form.
+int64_t mul_mat_least_workspace(int type, int64_t n_rows, int64_t k, int64_t m);
+
 // Rows row0 .. row0 + rows - 1 of a planar n_rows x k matrix to bf16 (dequant.hip).
 int dequant_rows(int type, const void* w, int64_t n_rows, int64_t k, int64_t row0, int64_t rows, uint16_t* out,
                  int64_t ld_out, hipStream_t s);

@@ -16,7 +16,9 @@
 //  - the llama.cpp shim's tensor conversion, restated from INTEGRATION.md
 //    over a minimal ggml_tensor, on storage filled with garbage first: a row
 //    view and a whole-expert view of a weight through spiral_supports_op
-//    (which reads view_src before any buffer check) and the size query.
+//    (which reads view_src before any buffer check) and the size query;
+//  - the growth of a backend's scratch on an allocator with a limit: what a
+//    graph wants, what it cannot do without, and what the scratch had before.
 // Any sanitizer report aborts the program (-fno-sanitize-recover=all); a
 // failed expectation prints the case and makes the exit status nonzero.
 #include <cstdint>
@@ -26,6 +28,7 @@
 #include <limits>
 #include <vector>
 
+#include "scratch.h"
 #include "spiral_ggml.h"
 #include "spiral_quants.h"
 
@@ -503,6 +506,42 @@ void check_shim() {
   }
 }
 
+// An allocator with `room` bytes, checked for leaks and double releases by the
+// sanitizer and by its count.
+void check_scratch() {
+  struct Heap {
+    size_t room, used = 0;
+    int live = 0;
+  } heap{1000};
+  spiral::Scratch s;
+  const auto alloc = [&](size_t n) -> void* {
+    if (n > heap.room - heap.used) return nullptr;
+    heap.used += n;
+    ++heap.live;
+    return std::malloc(n);
+  };
+  const auto release = [&](void* p) {
+    heap.used -= s.size;
+    --heap.live;
+    std::free(p);
+  };
+  const auto grown = [&](size_t need, size_t least) { return spiral::grow(s, need, least, alloc, release); };
+  EXPECT(grown(0, 0) && s.size == 0 && heap.live == 0, "scratch: nothing asked");
+  EXPECT(grown(300, 100) && s.size == 300 && heap.used == 300, "scratch: all of it");
+  EXPECT(grown(200, 200) && s.size == 300, "scratch: kept");
+  EXPECT(grown(1000, 100) && s.size == 1000 && heap.used == 1000, "scratch: the old memory goes first");
+  heap.room = 400;  // room for less than it has, from the next growth on
+  heap.used = 1000;
+  EXPECT(grown(900, 900) && s.size == 1000, "scratch: no growth, no call");
+  release(s.base);
+  s = spiral::Scratch{};
+  EXPECT(grown(2000, 350) && s.size == 350 && heap.live == 1, "scratch: the least");
+  EXPECT(grown(2000, 100) && s.size == 350 && heap.live == 1, "scratch: no less than before");
+  EXPECT(!grown(2000, 500) && s.base == nullptr && s.size == 0 && heap.live == 0 && heap.used == 0, "scratch: neither");
+  EXPECT(grown(500, 400) && s.size == 400, "scratch: after a failure");
+  EXPECT(!grown(500, 500) && heap.live == 0, "scratch: the least is all of it");
+}
+
 }  // namespace
 
 int main() {
@@ -513,6 +552,8 @@ int main() {
   std::printf("oracle and CPU-baseline checks done (%d failures so far)\n", g_failures);
   check_shim();
   std::printf("shim checks done (%d failures so far)\n", g_failures);
+  check_scratch();
+  std::printf("scratch checks done (%d failures so far)\n", g_failures);
   check_validation();
   std::printf("validation checks done: %d failures\n", g_failures);
   return g_failures == 0 ? 0 : 1;
