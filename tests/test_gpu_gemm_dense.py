@@ -115,3 +115,18 @@ def test_bf16_error_is_the_roundings(cuda, m, n, k):
     assert not torch.equal(y, fused)
     rms = [float((a.double() - ref).square().mean().sqrt()) for a in (y, fused)]
     assert rms[0] <= (1 + 1e-6) * rms[1], rms
+
+
+# 20 k steps: prologue, steady state with its load counts, F32 flushes (every 5
+# steps) and tail. The sizes are the smallest that the tile estimate gives to
+# 128 x 128, 256 x 128, x 160, x 192, x 224 and x 256 (F32 stops at 160).
+@pytest.mark.parametrize("m,n", [(257, 5454), (257, 10883), (513, 10883), (513, 13628), (769, 12347), (769, 14360)])
+@pytest.mark.parametrize("out_dtype,tol", [(torch.bfloat16, REL_TOL), (torch.float32, REL_TOL_EXACT_W)])
+def test_dense_tiles_long_rows(cuda, m, n, out_dtype, tol):
+    qtype, k = O.Q6_K, 1280
+    assert takes_dense(qtype, m, n, k)
+    w = ops.to_planar(qtype, dev_u8(synth.make_weights(qtype, n, k, 250), cuda), n, k)
+    x = dev_bf16(synth.make_x(m, k, 251), cuda)
+    y = ops.mul_mat(qtype, w, n, k, x, out_dtype=out_dtype)
+    ref = x.double() @ ops.dequant(qtype, w, n, k).double().t()
+    assert rel_err(y.float().cpu().numpy(), ref.cpu().numpy()) <= tol
