@@ -8,8 +8,8 @@
 // costs less than repeating it.
 //
 // dense_kernel: one workgroup of 8 waves per BM x BN tile (BM = 64 MF, BN =
-// 32 NF), k steps of 64, two LDS stages (128 KiB at 256 x 256, one workgroup a
-// CU, two waves a SIMD).
+// 32 NF), k steps of 64, two or three LDS stages of each operand (Stages; 160 KiB
+// at 256 x 256), one workgroup a CU, two waves a SIMD.
 //  - Staging: buffer loads straight into LDS, 1 KiB an instruction: 8 rows of
 //    128 bytes, so a lane group of 8 reads one whole line. The 16-byte chunks
 //    of a row are stored permuted (chunk c of row r at c ^ (r / 2 % 8)) so that
@@ -26,15 +26,14 @@
 //    at a time between MFMAs: issued together they fill their queues, and the
 //    wave's next MFMA waits behind them.
 //
-// Measured, Q4_K 14336 x 4096, 2048 rows of x, bf16 out: 361 us fused, 230 us
-// here (28 us the dequantization, 196-202 us the product, 1.05 PFLOP/s; a dense
+// Measured, Q4_K 14336 x 4096, 2048 rows of x, bf16 out: 344 us fused, 217 us
+// here (28 us the dequantization, 190 us the product, 1.27 PFLOP/s; a dense
 // library product of this shape takes 209 us). What bounds it: with the direct
 // loads left out the product takes 172 us, at the 1.95 GHz the clock falls to
 // under this load; with the MFMAs and LDS reads left out, 174 us. The loads are
 // bound by the lines a CU keeps in flight (about 80) against the latency of
 // filling L2: reading four k steps over and over, from L2, they take 86 us.
-// More stages at 128 x 128, k-sliced weights and plain stores of the
-// dequantized weights made no difference.
+// K-sliced weights and plain stores of the dequantized weights made no difference.
 #include <algorithm>
 #include <type_traits>
 
@@ -60,15 +59,15 @@ __device__ __forceinline__ uint32_t xcd_order(uint32_t b, uint32_t grid) {
 }
 
 // Bytes of an X and a W stage (W rows rounded up to whole loads by all waves),
-// and how many of each LDS holds: up to five where both fit three times, else
-// two of X and two or three of W.
+// and how many of each LDS holds: three where both fit, else two of X and, where
+// they fit, three of W. (4096 x 4096, 768 rows, 128 x 128 tiles: two of X and three
+// of W 60 us, three of both 50.8, five 50.9.)
 constexpr int kLdsBytes = 160 * 1024;
 template <int MF, int NF>
 struct Stages {
   static constexpr int kX = 64 * MF * kRowBytes, kW = 64 * ((NF + 1) / 2) * kRowBytes;
-  static constexpr int kBoth = std::min(5, kLdsBytes / (kX + kW));
-  static constexpr int kNX = kBoth >= 3 ? kBoth : 2;
-  static constexpr int kNW = kBoth >= 3 ? kBoth : 2 * kX + 3 * kW <= kLdsBytes ? 3 : 2;
+  static constexpr int kNX = 3 * (kX + kW) <= kLdsBytes ? 3 : 2;
+  static constexpr int kNW = kNX * kX + 3 * kW <= kLdsBytes ? 3 : 2;
   static constexpr int kBytes = kNX * kX + kNW * kW;
 };
 
