@@ -449,10 +449,9 @@ bool fusable_glu_split(const spiral_cgraph* graph, int32_t i) {
   return true;
 }
 
-// Where node i, a producer of F32 rows, leaves them as bf16 too: the start of
-// the scratch, if the next node multiplies them (their conversion costs a
-// launch of its own, 2.7 us and its gap for one row). Empty tensors and others
-// that the product would read in place have none.
+// Where node i, a producer of rows, leaves them as bf16 too: the start of the
+// scratch, if they are F32 and the next node multiplies them (their conversion
+// costs a launch of its own, 2.7 us and its gap for one row).
 uint16_t* copy_for_next(const spiral_backend* be, const spiral_cgraph* graph, int32_t i) {
   const spiral_tensor* t = graph->nodes[i];
   if (i + 1 >= graph->n_nodes || t->type != SPIRAL_TYPE_F32) return nullptr;

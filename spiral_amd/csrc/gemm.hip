@@ -367,7 +367,10 @@ int64_t packed_bytes(int64_t m, int64_t k) { return ceil_div(std::min(m, chunk_r
 // times the bytes of the packed x: long rows (a down projection) split, square
 // projections do not. Q5_K, us, one range against the split: 4096 x 14336, 77 rows
 // (64 tiles, four ranges) 73 and 31, 250 rows (two) 79 and 52; 2048 x 8192, 77
-// rows 45 and 21; 1024 x 4096, 250 rows 28 and 21.
+// rows 45 and 21; 1024 x 4096, 250 rows 28 and 21. The bounds on the sums and on a
+// range keep square projections at one range though they would gain too, at 17
+// rows more than at 128 (one, two and four ranges): 4096 x 4096, 17 rows 26, 19 and
+// 16, 128 rows 27, 22 and 22; 5120 x 5120, 77 rows 31, 24 and 29.
 int64_t k_splits(int64_t m, int64_t n_rows, int64_t k) {
   if (m > chunk_rows(k) || n_rows % 4 != 0) return 1;
   const int64_t tiles = ceil_div(m, kBM) * ceil_div(n_rows, kBN);

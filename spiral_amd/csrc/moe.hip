@@ -2,12 +2,15 @@
 // quantized, expert-stacked weights).
 //
 // Routing: at decode sizes (at most kFusedPairs (token, slot) pairs) each
-// moe_kernel workgroup scans the ids for its own expert into LDS, and the
-// workgroups of expert 0 also write the zero rows of pairs whose id is out
-// of range: one launch. Larger batches first run route_kernel (one
-// workgroup): a counting sort of the pairs by expert id into per-expert
-// lists in the caller's workspace, pairs with an out-of-range id getting a
-// zero output row.
+// workgroup of the two kernels here scans the ids for its own expert into LDS,
+// and the workgroups of expert 0 also write the zero rows of pairs whose id is
+// out of range: one launch. Larger batches, and the tiled form at any size, first
+// run route_kernel (one workgroup): a counting sort of the pairs by expert id into
+// per-expert lists in the caller's workspace, pairs with an out-of-range id getting
+// a zero output row.
+//
+// Batches of tens of tokens an expert run moe_tile_kernel (moe_tile.hip), where
+// its format and their count fit (moe_tile_fits). The others:
 //
 // moe_stream_kernel (k <= kStreamMaxK, every shape the decode path meets):
 //     a few workgroups per expert, each over a contiguous range of 16-row
@@ -1532,8 +1535,9 @@ void* moe_static_scratch(int& rc) {
 }
 
 // Arguments validated by the caller. glu_op < 0: plain MUL_MAT_ID; otherwise
-// the fused GLU form (n_rows = 2F even), which only the streaming form
-// implements (k <= kStreamMaxK and y below 2 GiB, else SPIRAL_ERR_SHAPE):
+// the fused GLU form (n_rows = 2F even), which the streaming and the tiled form
+// implement (k <= kStreamMaxK and y below 2 GiB, the streaming form's limits, for
+// both: else SPIRAL_ERR_SHAPE):
 // gate rows [0, F) and up rows [F, 2F) of each expert matrix, or, with w_up
 // set (ggml's split form), the F rows of w and of w_up, both at
 // expert_stride.

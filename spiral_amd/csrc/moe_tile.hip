@@ -15,7 +15,8 @@
 //    reads spread over the banks.
 //  - Wave s forms MFMA s of every 128-wide step (moe_piece.h) for all 96 rows:
 //    each (row, token) sum is the streaming form's four chains added in its
-//    order, so both forms give the same bits. (The eight elements of a lane may
+//    order, so both forms give the same bits (moe_kernel, which takes small batches
+//    past k = 4096, sums in another order). (The eight elements of a lane may
 //    come in any order and the two operands may change places: both measured
 //    bit-equal on gfx950; elements moved between lane groups are not.) Every code
 //    and every x element is then read from LDS by one wave only.
@@ -376,9 +377,14 @@ int launch_tile(const void* w, const void* w_up, int64_t expert_stride, int64_t 
 // its weights ahead better: gate_up and down of 128 experts, 2048 / 768, us,
 // streaming against this form at 17, 20 and 24 tokens an expert (its passes take
 // 32): Q4_K 142 and 166, 145 and 167, 237 and 176; Q4_0 123 and 160, 162 and 164,
-// 199 and 173; IQ4_XS 159 and 189, 210 and 185, 267 and 194. Past k = 2304 its
-// passes stay at 16: 60 experts, 3072 / 1536, 13 tokens: Q4_K 310 and 221, Q4_0
-// 246 and 203, IQ4_XS 264 and 239.
+// 199 and 173; IQ4_XS 159 and 189, 210 and 185, 267 and 194. The two products apart
+// at 20 and 24: Q5_K 172 and 114, 173 and 116 (gate_up), 43 and 65, 71 and 67
+// (down); IQ4_NL 95 and 101, 167 and 106, 42 and 59, 69 and 63. Past k = 2304 the
+// streaming form's passes stay at 16: 60 experts, 3072 / 1536, 13 tokens: Q4_K 310
+// and 221, Q4_0 246 and 203, IQ4_XS 264 and 239; one product at 13: Q5_K 60 experts
+// of 2048 x 2560 128 and 91, 16 of 4096 x 4096 102 and 79, 8 of 4096 x 14336 177
+// and 152, IQ4_NL 87 and 82, 82 and 71, 167 and 138; at 10 Q4_K 1.57 times the
+// streaming form's time in 16 of 4096 x 4096.
 //
 // short_rows: a product without GLU whose rows leave LDS for the streaming form's
 // passes of 64 tokens. It stays with that form while the average expert fills at
